@@ -8,8 +8,8 @@
 // MI355X design:
 //  * One workgroup per output tile, chosen by row count (gemm_plan): 32, 64 or 128 rows by
 //    128 columns on 4 waves for decode-sized M, 256 x 128 on 8 waves up to 1024 rows,
-//    256 x 256 on 8 waves above.  A wave owns a block of v_mfma_f32_32x32x16_bf16 tiles
-//    (4 x 2 of them in the large tiles: 128 fp32 accumulators per lane).
+//    256 x 256 on 4 waves above.  A wave owns a block of v_mfma_f32_32x32x16_bf16 tiles
+//    (16 x 16 x 32 in the 256 x 256 tile).
 //  * Both operand tiles of a k step (64 or 32 wide) move global -> LDS by DMA
 //    (global_load_lds_dwordx4, 1 KiB per wave instruction) into a ring of 2 to 8 steps,
 //    as deep as 160 KiB of LDS allows, every slot in flight.  The step's one barrier sits
@@ -25,6 +25,8 @@
 #include "fqa_append_math.h"
 #include "fqa_common.h"
 #include "fqa_gemm_internal.h"
+
+#include <type_traits>
 
 namespace fqa {
 namespace {
@@ -56,8 +58,36 @@ struct Tile {
   static_assert(kRing * kStage <= 160 * 1024, "LDS");
   static_assert((kRing - 1) * (kDmaA + kDmaB) < 64, "vmcnt");
   __device__ static int swz(int r) { return kChunks == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); }
+  // Accumulator block (rb, cb) of wave (wm, wn): the MFMAs compute the transposed block (W
+  // fragments as the row operand), so a lane holds one row of the tile and kQuads runs of 4
+  // consecutive columns.
+  typedef float16_t Block;
+  static constexpr int kQuads = 4, kRowLanes = 32;
+  __device__ static int row(int wm, int rb, int lane) { return (wm * kTM + rb) * 32 + (lane & 31); }
+  __device__ static int col(int wn, int cb, int q, int lane) {
+    return (wn * kTN + cb) * 32 + 8 * q + 4 * (lane >> 5);
+  }
 };
-using TileL = Tile<2, 4, 4, 2, 2, 64>;  // 256 x 256 on 8 waves: prefill-sized M
+// 256 x 256 on 4 waves (gemm_quad_kernel): prefill-sized M.  Each operand tile is two
+// halves of 128 rows; a wave's 128 x 128 outputs are four 64 x 64 quadrants, one per (x
+// half, W half), of 16 x 16 blocks.
+struct TileL {
+  static constexpr int kWM = 2, kWN = 2, kTM = 8, kTN = 8;
+  static constexpr int kBK = 64, kPitch = 128;
+  static constexpr int kBM = 256, kBN = 256;
+  static constexpr int kHalf = 128 * kPitch;  // one operand half: 128 rows x 64 k, 16 KiB
+  static constexpr int kRing = 2, kStage = 4 * kHalf;
+  static constexpr int kWaves = kWM * kWN, kThreads = 64 * kWaves;
+  __device__ static int swz(int r) { return (r >> 1) & 7; }
+  typedef float4_t Block;
+  static constexpr int kQuads = 1, kRowLanes = 16;
+  __device__ static int row(int wm, int rb, int lane) {
+    return (rb >> 2) * 128 + wm * 64 + (rb & 3) * 16 + (lane & 15);
+  }
+  __device__ static int col(int wn, int cb, int, int lane) {
+    return (cb >> 2) * 128 + wn * 64 + (cb & 3) * 16 + 4 * (lane >> 4);
+  }
+};
 using TileL8 = Tile<4, 2, 2, 2, 3>;     // 256 x 128 on 8 waves: 129..1024 rows
 using TileM = Tile<2, 2, 2, 2, 5>;      // 128 x 128
 using TileS = Tile<1, 4, 2, 1, 6>;      // 64 x 128
@@ -133,13 +163,153 @@ constexpr int kTilePitch = T::kBN * 2 + 16;
 template <class T>
 constexpr int kAppendLds = T::kBM * kTilePitch<T> + T::kBM * 8;
 template <class T, bool kAppend>
-constexpr int kGemmLds = kAppend && kAppendLds<T> > T::kRing * T::kStage
+constexpr int kGemmLds = (kAppend || T::kBN == 256) && kAppendLds<T> > T::kRing * T::kStage
                              ? kAppendLds<T>
                              : T::kRing * T::kStage;
 
+// The tile rounded to bf16 in LDS, row r at r * kTilePitch (every wave's reads of the operand
+// ring are done first; on return every wave sees the tile).
 template <class T>
-__device__ void append_epilogue(const GemmArgs& a, char* lds, const float16_t (&acc)[T::kTM][T::kTN],
+__device__ __forceinline__ void stage_tile(char* lds, const typename T::Block (&acc)[T::kTM][T::kTN],
+                                           int wm, int wn, int lane) {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's reads of the ring are done
+  barrier();                           // ... and every wave's: the LDS is free
+#pragma unroll
+  for (int rb = 0; rb < T::kTM; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < T::kTN; ++cb)
+#pragma unroll
+      for (int q = 0; q < T::kQuads; ++q)
+        *reinterpret_cast<uint2*>(lds + T::row(wm, rb, lane) * kTilePitch<T> +
+                                  T::col(wn, cb, q, lane) * 2) =
+            make_uint2(pack_bf16x2(acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1]),
+                       pack_bf16x2(acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]));
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  barrier();
+}
+
+template <class T>
+__device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::Block (&acc)[T::kTM][T::kTN],
                                 int row0, int col0, int wm, int wn, int w, int lane);
+
+// What a workgroup does with its tile's accumulators.
+template <class T, bool kF32Out, bool kPartial, bool kArgmax, bool kAppend>
+__device__ __forceinline__ void tile_epilogue(const GemmArgs& a, char* lds,
+                                              const typename T::Block (&acc)[T::kTM][T::kTN], int row0,
+                                              int col0, int tn, int sp, int wm, int wn, int w,
+                                              int lane) {
+  if constexpr (kAppend) {
+    append_epilogue<T>(a, lds, acc, row0, col0, wm, wn, w, lane);
+    return;
+  }
+  if constexpr (kArgmax) {
+    // per row of the tile: the largest value and its column (ties in the reference's greedy
+    // order, greedy_key), over this lane's values, then the wave's other lanes of the same
+    // row, then the tile's kWN column waves through LDS (free once every wave's reads are
+    // done)
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    barrier();
+    float* sv = reinterpret_cast<float*>(lds);
+    int* si = reinterpret_cast<int*>(lds + T::kBM * T::kWN * 4);
+#pragma unroll
+    for (int rb = 0; rb < T::kTM; ++rb) {
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
+      uint32_t bk = 0xffffffffu;
+#pragma unroll
+      for (int cb = 0; cb < T::kTN; ++cb)
+#pragma unroll
+        for (int q = 0; q < T::kQuads; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = acc[rb][cb][4 * q + e];
+            const int n = col0 + T::col(wn, cb, q, lane) + e;
+            const uint32_t k = greedy_key(n);
+            if (v > bv || (v == bv && k < bk)) {
+              bv = v;
+              bi = n;
+              bk = k;
+            }
+          }
+#pragma unroll
+      for (int o = T::kRowLanes; o < kWave; o *= 2) {
+        const float ov = __shfl_xor(bv, o, kWave);
+        const int oi = __shfl_xor(bi, o, kWave);
+        if (ov > bv || (ov == bv && greedy_key(oi) < greedy_key(bi))) {
+          bv = ov;
+          bi = oi;
+        }
+      }
+      const int r = T::row(wm, rb, lane);  // row within the tile
+      if (lane < T::kRowLanes) {
+        sv[r * T::kWN + wn] = bv;
+        si[r * T::kWN + wn] = bi;
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    barrier();
+    for (int r = threadIdx.x; r < T::kBM; r += T::kThreads) {
+      const int m = row0 + r;
+      if (m >= a.M) continue;
+      float bv = sv[r * T::kWN];
+      int bi = si[r * T::kWN];
+      for (int k = 1; k < T::kWN; ++k)
+        if (sv[r * T::kWN + k] > bv ||
+            (sv[r * T::kWN + k] == bv && greedy_key(si[r * T::kWN + k]) < greedy_key(bi))) {
+          bv = sv[r * T::kWN + k];
+          bi = si[r * T::kWN + k];
+        }
+      // row-major by row, so the reduction reads each row's maxima contiguously (these
+      // scattered 4-byte stores are a few hundred per tile of a long kernel)
+      a.amax_v[(long long)m * a.n_tiles + tn] = bv;
+      a.amax_i[(long long)m * a.n_tiles + tn] = bi;
+    }
+    return;
+  }
+
+  if constexpr (T::kBN == 256 && !kPartial && !kF32Out) {
+    // Stored straight from the accumulators, every instruction touches 16 rows with 32 bytes
+    // each, ~4 address cycles per row (7 us per tile); the tile goes through LDS instead and
+    // out as whole 512-byte rows, two per store.
+    stage_tile<T>(lds, acc, wm, wn, lane);
+    uint16_t* y = static_cast<uint16_t*>(a.y) + col0;
+    const bool wide = (a.ldy & 7) == 0;  // rows start on 16 bytes
+    for (int r0 = 2 * w; r0 < T::kBM; r0 += 2 * T::kWaves) {
+      const int r = r0 + (lane >> 5), m = row0 + r;
+      const uint4 v = *reinterpret_cast<const uint4*>(lds + r * kTilePitch<T> + (lane & 31) * 16);
+      if (m >= a.M) continue;
+      uint16_t* d = y + m * a.ldy + (lane & 31) * 8;
+      if (wide) {
+        *reinterpret_cast<uint4*>(d) = v;
+      } else {
+        *reinterpret_cast<uint2*>(d) = make_uint2(v.x, v.y);
+        *reinterpret_cast<uint2*>(d + 4) = make_uint2(v.z, v.w);
+      }
+    }
+    return;
+  }
+  // one 16-byte (fp32) or 8-byte (bf16) store per run of 4 columns
+#pragma unroll
+  for (int rb = 0; rb < T::kTM; ++rb) {
+    const int m = row0 + T::row(wm, rb, lane);
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int cb = 0; cb < T::kTN; ++cb)
+#pragma unroll
+      for (int q = 0; q < T::kQuads; ++q) {
+        const int n = col0 + T::col(wn, cb, q, lane);
+        const float4 v = make_float4(acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1],
+                                     acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]);
+        if (kPartial)
+          *reinterpret_cast<float4*>(a.part + ((long long)sp * a.M + m) * a.N + n) = v;
+        else if (kF32Out)
+          *reinterpret_cast<float4*>(static_cast<float*>(a.y) + m * a.ldy + n) = v;
+        else
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + m * a.ldy + n) =
+              make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+      }
+  }
+}
 
 template <class T, bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
 __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
@@ -256,96 +426,182 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
     }
   }
 
-  if constexpr (kAppend) {
-    append_epilogue<T>(a, lds, acc, row0, col0, wm, wn, w, lane);
-    return;
-  }
-  if constexpr (kArgmax) {
-    // per row of the tile: the largest value and its column (ties in the reference's greedy order, greedy_key), over
-    // this lane's values, then lane ^ 32 (the other column half of the same row), then
-    // the tile's kWN column waves through LDS (free once every wave's reads are done)
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    barrier();
-    float* sv = reinterpret_cast<float*>(lds);
-    int* si = reinterpret_cast<int*>(lds + T::kBM * T::kWN * 4);
-#pragma unroll
-    for (int rb = 0; rb < T::kTM; ++rb) {
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-      uint32_t bk = 0xffffffffu;
-#pragma unroll
-      for (int cb = 0; cb < T::kTN; ++cb)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float v = acc[rb][cb][4 * q + e];
-            const int n = col0 + (wn * T::kTN + cb) * 32 + 8 * q + 4 * (lane >> 5) + e;
-            const uint32_t k = greedy_key(n);
-            if (v > bv || (v == bv && k < bk)) {
-              bv = v;
-              bi = n;
-              bk = k;
-            }
-          }
-      const float ov = __shfl_xor(bv, 32, kWave);
-      const int oi = __shfl_xor(bi, 32, kWave);
-      if (ov > bv || (ov == bv && greedy_key(oi) < greedy_key(bi))) {
-        bv = ov;
-        bi = oi;
-      }
-      const int r = (wm * T::kTM + rb) * 32 + (lane & 31);  // row within the tile
-      if (lane < 32) {
-        sv[r * T::kWN + wn] = bv;
-        si[r * T::kWN + wn] = bi;
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    barrier();
-    for (int r = threadIdx.x; r < T::kBM; r += T::kThreads) {
-      const int m = row0 + r;
-      if (m >= a.M) continue;
-      float bv = sv[r * T::kWN];
-      int bi = si[r * T::kWN];
-      for (int k = 1; k < T::kWN; ++k)
-        if (sv[r * T::kWN + k] > bv ||
-            (sv[r * T::kWN + k] == bv && greedy_key(si[r * T::kWN + k]) < greedy_key(bi))) {
-          bv = sv[r * T::kWN + k];
-          bi = si[r * T::kWN + k];
-        }
-      // row-major by row, so the reduction reads each row's maxima contiguously (these
-      // scattered 4-byte stores are a few hundred per tile of a long kernel)
-      a.amax_v[(long long)m * a.n_tiles + tn] = bv;
-      a.amax_i[(long long)m * a.n_tiles + tn] = bi;
-    }
-    return;
-  }
+  tile_epilogue<T, kF32Out, kPartial, kArgmax, kAppend>(a, lds, acc, row0, col0, tn, sp, wm, wn, w,
+                                                        lane);
+}
 
-  // The MFMAs compute the transposed block (W fragments as the 32-row operand), so
-  // accumulator (rb, cb) registers 4q..4q+3 of lane hold row 32 rb + lane % 32 and the 4
-  // consecutive columns 32 cb + 8 q + 4 (lane / 32) + 0..3 of the wave's block: one
-  // 16-byte (fp32) or 8-byte (bf16) store each, a quarter of the store instructions of
-  // a row-per-register layout
+// The 256 x 256 tile: one wave per SIMD, each 128 x 128.  A step is 64 k of both operands,
+// four 16 KiB halves (x rows 0-127 and 128-255: A0, A1; W rows likewise: B0, B1), double
+// buffered, and four phases of 32 MFMAs per wave, one per quadrant, in the order (A0,B0)
+// (A0,B1) (A1,B1) (A1,B0).
+//  * Every phase reads from LDS the half the next phase adds (B1, A1, A0(t+1), B0(t+1)), and
+//    issues the DMA of one half (A1(t+1), A0(t+2), B0(t+2), B1(t+2)), spread between its
+//    MFMAs, so no wait sits in front of an MFMA and a half has 3 phases or more to land.
+//  * Two barriers per step, each behind a vmcnt that leaves the newest three halves in
+//    flight: after phase 2 A0(t+1) and B0(t+1) are in LDS for every wave, after phase 4
+//    B1(t+1) and A1(t+1).  A half's slot is refilled only after a barrier that follows every
+//    wave's last use of it: fragments are consumed by MFMAs before the barrier, except
+//    A0(t+1)'s, which the lgkmcnt before the second barrier waits for (B0(t+1)'s 8 are
+//    newer; they are consumed in phase 1 of t+1, a barrier before B0's refill).
+//  * What bounds it: the MFMAs at the clock the card holds under them (taking all DMA out of
+//    the loop changes 289 us to 292 on 8192 x 6144 x 4096, all waits and barriers to 282),
+//    then ~5 us per tile to start and to store.  16 x 16 x 32 MFMAs beat 32 x 32 x 16 here
+//    (289 against 313 us): 16-cycle steps leave the wave's other instructions more places to
+//    issue.  128 x 128 per wave reads each fragment for 8 MFMAs, 128 KiB of LDS reads per
+//    step against 192 KiB for the 8-wave tile this replaces.
+//  * 8192 rows, qkv / o_proj / gate_up / down: 325 / 221 / 1285 / 604 us (8 waves, 32 x 32
+//    MFMAs, the next step staged in one burst) -> 284 / 192 / 1158 / 545 us, 1.42-1.51
+//    PFLOP/s; 2048 rows 94 / 77 / 330 / 181 -> 85 / 71 / 298 / 160 us.
+template <bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
+__global__ void __launch_bounds__(TileL::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
+  using T = TileL;
+  __shared__ __attribute__((aligned(1024))) char lds[kGemmLds<T, kAppend>];
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w >> 1, wn = w & 1;
+  int tm, tn, sp;
+  tile_of(a, tm, tn, sp);
+  const int row0 = tm * T::kBM, col0 = tn * T::kBN;
+  const int nst = a.K / T::kBK;
+  const int n = (nst - sp + a.splits - 1) / a.splits;  // >= 1: splits <= steps
+  const long long kstride = (long long)a.splits * T::kBK;
+
+  // LDS: x halves of buffer b at b * 32 KiB + half * 16 KiB, W halves 64 KiB further on.
+  // Wave w's DMA instruction i of a half covers rows 32 w + 8 i + lane / 8; a lane fills LDS
+  // chunk lane % 8 of its row, so it reads global chunk (lane % 8) ^ swz(row).
+  constexpr int kB = 4 * T::kHalf, kDma = 4;
+  uint32_t off_a[2][kDma], off_b[2][kDma];
 #pragma unroll
-  for (int rb = 0; rb < T::kTM; ++rb) {
-    const int m = row0 + (wm * T::kTM + rb) * 32 + (lane & 31);
-    if (m >= a.M) continue;
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int cb = 0; cb < T::kTN; ++cb)
+    for (int i = 0; i < kDma; ++i) {
+      const int r = 32 * w + 8 * i + (lane >> 3);
+      const uint32_t c = ((lane & 7) ^ T::swz(r)) * 16;
+      const int gr = min(row0 + 128 * h + r, a.M - 1);
+      off_a[h][i] = (uint32_t)((long long)gr * a.ldx * 2) + c;
+      off_b[h][i] = (uint32_t)((long long)(col0 + 128 * h + r) * a.ldw * 2) + c;
+    }
+  const uint32_t dst0 = lds_base + w * (kDma * 1024);
+  auto stage_a = [&](const uint16_t* xs, int h, int buf, int i) {
+    dma16(xs, off_a[h][i], dst0 + (2 * buf + h) * T::kHalf + i * 1024);
+  };
+  auto stage_b = [&](const uint16_t* ws, int h, int buf, int i) {
+    dma16(ws, off_b[h][i], dst0 + kB + (2 * buf + h) * T::kHalf + i * 1024);
+  };
+  // the k steps' pointers: step 0, 1 (xs1, ws1) and, in the loop, t + 2; past the end the
+  // last step is staged again (never read), so that every wait count holds
+  const uint16_t* xs0 = a.x + (long long)sp * T::kBK;
+  const uint16_t* ws0 = a.w + (long long)sp * T::kBK;
+  const uint16_t* xs1 = n > 1 ? xs0 + kstride : xs0;
+  const uint16_t* ws1 = n > 1 ? ws0 + kstride : ws0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = col0 + (wn * T::kTN + cb) * 32 + 8 * q + 4 * (lane >> 5);
-        const float4 v = make_float4(acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1],
-                                     acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]);
-        if (kPartial)
-          *reinterpret_cast<float4*>(a.part + ((long long)sp * a.M + m) * a.N + n) = v;
-        else if (kF32Out)
-          *reinterpret_cast<float4*>(static_cast<float*>(a.y) + m * a.ldy + n) = v;
-        else
-          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + m * a.ldy + n) =
-              make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
-      }
+  for (int i = 0; i < kDma; ++i) stage_a(xs0, 0, 0, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_b(ws0, 0, 0, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_b(ws0, 1, 0, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_a(xs0, 1, 0, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_a(xs1, 0, 1, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_b(ws1, 0, 1, i);
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) stage_b(ws1, 1, 1, i);
+
+  // fragment (r, kk) of a half: row 64 * wave + 16 r + lane % 16, 16-byte chunk 4 kk + lane / 16
+  int pa[2], pb[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int c = ((4 * kk + (lane >> 4)) ^ T::swz(lane & 15)) * 16;
+    pa[kk] = (wm * 64 + (lane & 15)) * T::kPitch + c;
+    pb[kk] = kB + (wn * 64 + (lane & 15)) * T::kPitch + c;
   }
+  bf16x8 af[2][4][2], bf[2][4][2];  // [half][r][kk]
+  // fragment f = 4 kk + r of half h, in the buffer that pa / pb point at
+  auto read_a = [&](int h, int f) {
+    af[h][f & 3][f >> 2] = *reinterpret_cast<const bf16x8*>(lds + pa[f >> 2] + h * T::kHalf +
+                                                            (f & 3) * 16 * T::kPitch);
+  };
+  auto read_b = [&](int h, int f) {
+    bf[h][f & 3][f >> 2] = *reinterpret_cast<const bf16x8*>(lds + pb[f >> 2] + h * T::kHalf +
+                                                            (f & 3) * 16 * T::kPitch);
+  };
+  float4_t acc[T::kTM][T::kTN];
+#pragma unroll
+  for (int rb = 0; rb < T::kTM; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < T::kTN; ++cb) acc[rb][cb] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  // One phase: the 32 MFMAs of quadrant (x half i, W half j), kk outermost; between(g) places
+  // fragment reads and DMA instructions after each pair g.
+  auto phase = [&](int i, int j, auto&& between) {
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      const int kk = q >> 4, r = (q >> 2) & 3, c = q & 3;
+      acc[4 * i + r][4 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          bf[j][c][kk], af[i][r][kk], acc[4 * i + r][4 * j + c], 0, 0, 0);
+      if (q & 1) between(q >> 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  wait_vm<3 * kDma>();  // step 0
+  barrier();
+#pragma unroll
+  for (int f = 0; f < 8; ++f) read_a(0, f);
+#pragma unroll
+  for (int f = 0; f < 8; ++f) read_b(0, f);
+  for (int t = 0; t < n; ++t) {
+    const int buf = t & 1;
+    const bool more = t + 2 < n;
+    const uint16_t* xs2 = more ? xs1 + kstride : xs1;
+    const uint16_t* ws2 = more ? ws1 + kstride : ws1;
+    phase(0, 0, [&](int g) {
+      if (g < 8) read_b(1, g);
+      if ((g & 3) == 1) stage_a(xs1, 1, buf ^ 1, g >> 2);
+    });
+    phase(0, 1, [&](int g) {
+      if (g < 8) read_a(1, g);
+      if ((g & 3) == 1) stage_a(xs2, 0, buf, g >> 2);
+    });
+    wait_vm<3 * kDma>();  // A0(t+1), B0(t+1)
+    barrier();
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {  // the other buffer
+      pa[kk] ^= 2 * T::kHalf;
+      pb[kk] ^= 2 * T::kHalf;
+    }
+    phase(1, 1, [&](int g) {
+      if (g < 8) read_a(0, g);
+      if ((g & 3) == 1) stage_b(ws2, 0, buf, g >> 2);
+    });
+    phase(1, 0, [&](int g) {  // B0(t+1)'s fragments as B0(t)'s are used up
+      if (g >= 8 && g < 12) read_b(0, g - 8);
+      if (g == 15)
+#pragma unroll
+        for (int f = 4; f < 8; ++f) read_b(0, f);
+      if ((g & 3) == 1) stage_b(ws2, 1, buf, g >> 2);
+    });
+    wait_vm<3 * kDma>();  // B1(t+1), A1(t+1)
+    __builtin_amdgcn_s_waitcnt(0xC87F);  // lgkmcnt(8): A0(t+1) is read
+    barrier();
+    xs1 = xs2;
+    ws1 = ws2;
+  }
+  wait_vm<0>();  // the DMAs past the end: the LDS is reused or given back
+
+  // the epilogue's addresses are computed after the loop, not held in registers through it
+  int elane = lane, erow0 = row0, ecol0 = col0;
+  asm volatile("" : "+v"(elane), "+s"(erow0), "+s"(ecol0));
+  // ... and the accumulators stay in AGPRs up to here (VALU ops cannot read those: without
+  // this the allocator spreads the epilogue's copies into the loop and spills)
+#pragma unroll
+  for (int rb = 0; rb < T::kTM; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < T::kTN; ++cb) asm volatile("" : "+a"(acc[rb][cb]));
+  tile_epilogue<T, kF32Out, kPartial, kArgmax, kAppend>(a, lds, acc, erow0, ecol0, tn, sp, wm, wn, w,
+                                                        elane);
 }
 
 // The QKV projection's epilogue fused with the per-head norm + RoPE + paged append
@@ -359,7 +615,7 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
 //    token's column.
 // v is not written to qkv.  Rows at or past meta[FQA_META_ROWS] are not written.
 template <class T>
-__device__ void append_epilogue(const GemmArgs& a, char* lds, const float16_t (&acc)[T::kTM][T::kTN],
+__device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::Block (&acc)[T::kTM][T::kTN],
                                 int row0, int col0, int wm, int wn, int w, int lane) {
   constexpr int kTP = kTilePitch<T>;
   constexpr int kNH = T::kBN / kD;  // heads in the tile
@@ -373,20 +629,7 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const float16_t (&
     my_pos = p.positions[row0 + threadIdx.x];
     my_slot = p.slots[row0 + threadIdx.x];
   }
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's reads of the ring are done
-  barrier();                           // ... and every wave's: the LDS is free
-#pragma unroll
-  for (int rb = 0; rb < T::kTM; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < T::kTN; ++cb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = (wm * T::kTM + rb) * 32 + (lane & 31);
-        const int c = (wn * T::kTN + cb) * 32 + 8 * q + 4 * (lane >> 5);
-        *reinterpret_cast<uint2*>(lds + r * kTP + c * 2) =
-            make_uint2(pack_bf16x2(acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1]),
-                       pack_bf16x2(acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]));
-      }
+  stage_tile<T>(lds, acc, wm, wn, lane);
   if (threadIdx.x < T::kBM) {
     s_pos[threadIdx.x] = my_pos;
     s_slot[threadIdx.x] = my_slot;
@@ -604,6 +847,11 @@ bool gemm_shape_ok(int M, int N, int K) {
 
 template <class T>
 void launch_argmax(const GemmArgs& a, hipStream_t st) {
+  if constexpr (std::is_same_v<T, TileL>) {
+    hipLaunchKernelGGL((gemm_quad_kernel<false, false, true>),
+                       dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
+    return;
+  } else
   hipLaunchKernelGGL((gemm_kernel<T, false, false, true>),
                      dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
 }
@@ -611,7 +859,14 @@ template <class T>
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t st) {
   const dim3 grid((unsigned)(a.m_tiles * a.n_tiles * a.splits));
   const dim3 block(T::kThreads);
-  if (a.splits > 1)
+  if constexpr (std::is_same_v<T, TileL>) {
+    if (a.splits > 1)
+      hipLaunchKernelGGL((gemm_quad_kernel<false, true>), grid, block, 0, st, a);
+    else if (f32)
+      hipLaunchKernelGGL((gemm_quad_kernel<true, false>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((gemm_quad_kernel<false, false>), grid, block, 0, st, a);
+  } else if (a.splits > 1)
     hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, block, 0, st, a);
   else if (f32)
     hipLaunchKernelGGL((gemm_kernel<T, true, false>), grid, block, 0, st, a);
@@ -679,7 +934,7 @@ int gemm_launch_partials(const void* x, int64_t ldx, const void* w, int64_t ldw,
     a.app = *app;
     const dim3 grid((unsigned)(a.m_tiles * a.n_tiles));
     if (p.tile == 0)
-      hipLaunchKernelGGL((gemm_kernel<TileL, false, false, false, true>), grid,
+      hipLaunchKernelGGL((gemm_quad_kernel<false, false, false, true>), grid,
                          dim3(TileL::kThreads), 0, st, a);
     else
       hipLaunchKernelGGL((gemm_kernel<TileL8, false, false, false, true>), grid,

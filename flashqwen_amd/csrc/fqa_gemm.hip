@@ -6,19 +6,17 @@
 // both K-contiguous (the reference's weight layout), y is [M, N].
 //
 // MI355X design:
-//  * One workgroup per output tile, chosen by row count (gemm_plan): 32, 64 or 128 rows by
-//    128 columns on 4 waves for decode-sized M, 256 x 128 on 8 waves up to 1024 rows,
-//    256 x 256 on 4 waves above.  A wave owns a block of v_mfma_f32_32x32x16_bf16 tiles
-//    (16 x 16 x 32 in the 256 x 256 tile).
-//  * Both operand tiles of a k step (64 or 32 wide) move global -> LDS by DMA
-//    (global_load_lds_dwordx4, 1 KiB per wave instruction) into a ring of 2 to 8 steps,
-//    as deep as 160 KiB of LDS allows, every slot in flight.  The step's one barrier sits
-//    before its last MFMAs, so the freed slot is refilled and the next step's first
-//    fragments are read while those MFMAs run.  A DMA lane's 16 bytes land at LDS byte
-//    16 * lane, so the bank swizzle (Tile::swz) is applied on the global side of the DMA.
-//  * Shapes with few tiles (decode steps) split K over `splits` workgroups per tile so
-//    that one round of workgroups fills the 256 CUs; each writes fp32 partials and a
-//    second kernel sums them into y (or a fused consumer reads them: fqa_qkv_proj_append).
+//  * Four kernels, chosen by a model of their times (gemm_plan):
+//    - gemm_quad_kernel: tiles of 256 x 256, 256 x 128 and 128 x 128 on 4 waves, one per SIMD;
+//    - gemm_slab_kernel: up to 96 x 64 outputs per workgroup for few rows, its waves dividing K
+//      and summing in LDS, so that decode steps fill the CUs without a second kernel;
+//    - gemm_kernel: 32 and 64 rows by 128 columns where W is wide enough to fill the CUs;
+//    - where the tiles alone still leave CUs idle, K is split over workgroups that leave fp32
+//      partials, which gemm_reduce_kernel sums (or fqa_qkv_proj_append's append kernel reads).
+//  * Both operands move global -> LDS by DMA (global_load_lds_dwordx4, 1 KiB per wave
+//    instruction: 8 rows x 128 bytes) into a ring of k steps, as deep as 160 KiB of LDS
+//    allows, every slot in flight.  A DMA lane's 16 bytes land at LDS byte 16 * lane, so the
+//    bank swizzle (swz) is applied on the global side of the DMA.
 //  * Workgroups are dealt to the 8 XCDs round robin; tile_of() renumbers them so that the
 //    workgroups on one XCD walk 8 m tiles per n tile and share W and x tiles in its L2.
 
@@ -68,30 +66,39 @@ struct Tile {
     return (wn * kTN + cb) * 32 + 8 * q + 4 * (lane >> 5);
   }
 };
-// 256 x 256 on 4 waves (gemm_quad_kernel): prefill-sized M.  Each operand tile is two
-// halves of 128 rows; a wave's 128 x 128 outputs are four 64 x 64 quadrants, one per (x
-// half, W half), of 16 x 16 blocks.
-struct TileL {
-  static constexpr int kWM = 2, kWN = 2, kTM = 8, kTN = 8;
+// The tiles of gemm_quad_kernel: 4 waves, 2 x 2.  Each operand tile is two halves (rows
+// 0 .. kBM/2 - 1 and the rest; W rows likewise) and a wave's kBM/2 x kBN/2 outputs are four
+// quadrants, one per (x half, W half), of kQM x kQN 16 x 16 blocks.
+template <int kBM_, int kBN_, int kRing_>
+struct Quad {
+  static constexpr int kBM = kBM_, kBN = kBN_, kRing = kRing_;
+  static constexpr int kWM = 2, kWN = 2, kQM = kBM / 64, kQN = kBN / 64;
+  static constexpr int kTM = 2 * kQM, kTN = 2 * kQN;
   static constexpr int kBK = 64, kPitch = 128;
-  static constexpr int kBM = 256, kBN = 256;
-  static constexpr int kHalf = 128 * kPitch;  // one operand half: 128 rows x 64 k, 16 KiB
-  static constexpr int kRing = 2, kStage = 4 * kHalf;
-  static constexpr int kWaves = kWM * kWN, kThreads = 64 * kWaves;
+  static constexpr int kHalfA = kBM / 2 * kPitch, kHalfB = kBN / 2 * kPitch;  // bytes per step
+  static constexpr int kStage = 2 * (kHalfA + kHalfB);
+  static constexpr int kWaves = 4, kThreads = 256;
+  static constexpr int kDmaA = kBM / 64, kDmaB = kBN / 64;  // DMA instructions per wave per half
+  static_assert(kRing >= 2 && kRing * kStage <= 160 * 1024, "LDS");
   __device__ static int swz(int r) { return (r >> 1) & 7; }
   typedef float4_t Block;
   static constexpr int kQuads = 1, kRowLanes = 16;
   __device__ static int row(int wm, int rb, int lane) {
-    return (rb >> 2) * 128 + wm * 64 + (rb & 3) * 16 + (lane & 15);
+    return (rb / kQM) * (kBM / 2) + wm * (kBM / 4) + (rb % kQM) * 16 + (lane & 15);
   }
   __device__ static int col(int wn, int cb, int, int lane) {
-    return (cb >> 2) * 128 + wn * 64 + (cb & 3) * 16 + 4 * (lane >> 4);
+    return (cb / kQN) * (kBN / 2) + wn * (kBN / 4) + (cb % kQN) * 16 + 4 * (lane >> 4);
   }
 };
-using TileL8 = Tile<4, 2, 2, 2, 3>;     // 256 x 128 on 8 waves: 129..1024 rows
-using TileM = Tile<2, 2, 2, 2, 5>;      // 128 x 128
-using TileS = Tile<1, 4, 2, 1, 6>;      // 64 x 128
-using TileT = Tile<1, 4, 1, 1, 8>;      // 32 x 128: a few decode rows
+template <class T>
+constexpr bool kIsQuad = false;
+template <int M, int N, int R>
+constexpr bool kIsQuad<Quad<M, N, R>> = true;
+using TileL = Quad<256, 256, 2>;
+using TileH = Quad<256, 128, 3>;
+using TileM = Quad<128, 128, 5>;
+using TileS = Tile<1, 4, 2, 1, 6>;  // 64 x 128
+using TileT = Tile<1, 4, 1, 1, 8>;  // 32 x 128: a few decode rows
 
 struct GemmArgs {
   const uint16_t* x;
@@ -114,6 +121,22 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t l
       :
       : "v"(off), "s"(base), "{m0}"(lds)
       : "memory");
+}
+// ... of W, with the non-temporal hint (kNT) where no other workgroup reads it: 1.2 GB
+// streamed by 256 workgroups 198 -> 176 us, 201 MB 41 -> 37.5 us (DMA alone); gate_up at 6
+// rows 42.8 -> 39.0 us.  With K split over workgroups it costs instead (6144 x 4096 at 64
+// rows 17.8 -> 19.3 us).
+template <bool kNT>
+__device__ __forceinline__ void dma16_w(const void* base, uint32_t off, uint32_t lds) {
+  if constexpr (kNT)
+    asm volatile(
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %1 nt"
+        :
+        : "v"(off), "s"(base), "{m0}"(lds)
+        : "memory");
+  else
+    dma16(base, off, lds);
 }
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -163,7 +186,7 @@ constexpr int kTilePitch = T::kBN * 2 + 16;
 template <class T>
 constexpr int kAppendLds = T::kBM * kTilePitch<T> + T::kBM * 8;
 template <class T, bool kAppend>
-constexpr int kGemmLds = (kAppend || T::kBN == 256) && kAppendLds<T> > T::kRing * T::kStage
+constexpr int kGemmLds = (kAppend || kIsQuad<T>) && kAppendLds<T> > T::kRing * T::kStage
                              ? kAppendLds<T>
                              : T::kRing * T::kStage;
 
@@ -191,6 +214,53 @@ __device__ __forceinline__ void stage_tile(char* lds, const typename T::Block (&
 template <class T>
 __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::Block (&acc)[T::kTM][T::kTN],
                                 int row0, int col0, int wm, int wn, int w, int lane);
+
+// K in four segments, begun at another one by workgroups that run side by side: in lockstep
+// at one k offset of rows a power of two apart they meet on the same HBM channels (DMA alone:
+// 201 MB by 256 workgroups 37.7 -> 31.3 us, by 192 40.4 -> 30.2; 67 MB 17.9 -> 11.8).  The
+// sums stay independent of where a workgroup begins, so equal columns give equal values: the
+// segments' sums a0..a3, in the order taken, add up as (a0 + a2) + (a1 + a3), which any
+// rotation leaves the same.
+struct Segments {
+  int n, start;  // steps, the first segment
+  __device__ int first() const { return start * n / 4; }  // its first step
+  __device__ int end(int taken) const {  // steps of the segments 0 .. taken, in the order taken
+    const int e = start + taken + 1;
+    return (e > 4 ? (e - 4) * n / 4 + n : e * n / 4) - first();
+  }
+};
+// Segment e (0..3 in the order taken) is complete in acc: kept in (or added to) sum[e & 1],
+// acc cleared for the next; after the last, acc is the total.
+template <int e, class B, int kM, int kN>
+__device__ __forceinline__ void close_segment(B (&sum)[2][kM][kN], B (&acc)[kM][kN]) {
+#pragma unroll
+  for (int rb = 0; rb < kM; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < kN; ++cb) {
+      if constexpr (e < 2)
+        sum[e][rb][cb] = acc[rb][cb];
+      else if constexpr (e == 2)
+        sum[0][rb][cb] += acc[rb][cb];
+      else
+        acc[rb][cb] = sum[0][rb][cb] + (sum[1][rb][cb] + acc[rb][cb]);
+      if constexpr (e < 3)
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(B) / 4); ++i) acc[rb][cb][i] = 0.f;
+    }
+}
+// steps(end) runs the steps up to `end`.
+template <class F, class B, int kM, int kN>
+__device__ __forceinline__ void run_segments(const Segments& segs, B (&acc)[kM][kN], F&& steps) {
+  B sum[2][kM][kN];
+  steps(segs.end(0));
+  close_segment<0>(sum, acc);
+  steps(segs.end(1));
+  close_segment<1>(sum, acc);
+  steps(segs.end(2));
+  close_segment<2>(sum, acc);
+  steps(segs.n);
+  close_segment<3>(sum, acc);
+}
 
 // What a workgroup does with its tile's accumulators.
 template <class T, bool kF32Out, bool kPartial, bool kArgmax, bool kAppend>
@@ -267,18 +337,19 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& a, char* lds,
     return;
   }
 
-  if constexpr (T::kBN == 256 && !kPartial && !kF32Out) {
+  if constexpr (kIsQuad<T> && !kPartial && !kF32Out) {
     // Stored straight from the accumulators, every instruction touches 16 rows with 32 bytes
     // each, ~4 address cycles per row (7 us per tile); the tile goes through LDS instead and
-    // out as whole 512-byte rows, two per store.
+    // out as whole rows of the tile.
     stage_tile<T>(lds, acc, wm, wn, lane);
     uint16_t* y = static_cast<uint16_t*>(a.y) + col0;
     const bool wide = (a.ldy & 7) == 0;  // rows start on 16 bytes
-    for (int r0 = 2 * w; r0 < T::kBM; r0 += 2 * T::kWaves) {
-      const int r = r0 + (lane >> 5), m = row0 + r;
-      const uint4 v = *reinterpret_cast<const uint4*>(lds + r * kTilePitch<T> + (lane & 31) * 16);
+    constexpr int kRowChunks = T::kBN / 8, kRows = kWave / kRowChunks;  // rows per store
+    for (int r0 = kRows * w; r0 < T::kBM; r0 += kRows * T::kWaves) {
+      const int r = r0 + lane / kRowChunks, c = lane % kRowChunks, m = row0 + r;
+      const uint4 v = *reinterpret_cast<const uint4*>(lds + r * kTilePitch<T> + c * 16);
       if (m >= a.M) continue;
-      uint16_t* d = y + m * a.ldy + (lane & 31) * 8;
+      uint16_t* d = y + m * a.ldy + c * 8;
       if (wide) {
         *reinterpret_cast<uint4*>(d) = v;
       } else {
@@ -311,9 +382,12 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& a, char* lds,
   }
 }
 
-template <class T, bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
+// The tiles of 32 and 64 rows, which stream W once (one row tile, no K split): gate_up at 6 /
+// 64 rows 45.5 / 47.5 -> 32.8 / 38.3 us with the segments and the non-temporal W loads,
+// lm_head at 2 rows 264 -> 193 us (6.5 TB/s).
+template <class T, bool kF32Out, bool kArgmax = false>
 __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kGemmLds<T, kAppend>];
+  __shared__ __attribute__((aligned(1024))) char lds[kGemmLds<T, false>];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -321,13 +395,9 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
   int tm, tn, sp;
   tile_of(a, tm, tn, sp);
   const int row0 = tm * T::kBM, col0 = tn * T::kBN;
-  // split sp takes k steps sp, sp + splits, sp + 2 splits, ...: the splits of a tile run
-  // side by side and read adjacent pieces of the same W rows
-  const int nst = a.K / T::kBK;
-  const int n_my = (nst - sp + a.splits - 1) / a.splits;
-  const int kstride = a.splits * T::kBK;
-  const uint16_t* xk = a.x + (long long)sp * T::kBK;
-  const uint16_t* wk = a.w + (long long)sp * T::kBK;
+  const int n_my = a.K / T::kBK;
+  const uint16_t* xk = a.x;
+  const uint16_t* wk = a.w;
 
   // DMA sources: wave w's instruction i covers rows kRowsPerDma (w kDmaA + i) + lane /
   // kChunks of the x tile (likewise of the W tile); lane fills LDS chunk lane % kChunks
@@ -346,13 +416,17 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
     off_b[i] = (uint32_t)((long long)(col0 + tr) * a.ldw * 2) + (dlc ^ T::swz(tr)) * 16;
   }
   // load q (0 .. kDmaA + kDmaB - 1) of this wave's share of the workgroup's j-th k step
+  const Segments segs{n_my, (int)(blockIdx.x >> 3) & 3};
+  const int rot = segs.first();
   auto issue_one = [&](int j, int q) {
     const uint32_t dst = lds_base + (j % T::kRing) * T::kStage;
+    j += rot;
+    if (j >= n_my) j -= n_my;
     if (q < T::kDmaA)
-      dma16(xk + (long long)j * kstride, off_a[q], dst + (w * T::kDmaA + q) * 1024);
+      dma16(xk + (long long)j * T::kBK, off_a[q], dst + (w * T::kDmaA + q) * 1024);
     else
-      dma16(wk + (long long)j * kstride, off_b[q - T::kDmaA],
-            dst + T::kABytes + (w * T::kDmaB + q - T::kDmaA) * 1024);
+      dma16_w<true>(wk + (long long)j * T::kBK, off_b[q - T::kDmaA],
+                     dst + T::kABytes + (w * T::kDmaB + q - T::kDmaA) * 1024);
   };
   auto issue = [&](int j) {
 #pragma unroll
@@ -396,65 +470,70 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
   wait_steps<kPer, T::kRing - 1>(min(T::kRing - 1, n_my - 1));
   barrier();  // step 0 landed for every wave
   read_frags(0, 0, 0);
-  for (int s = 0; s < n_my; ++s) {
+  int s = 0;
+  auto steps = [&](int end) {
+    for (; s < end; ++s) {
 #pragma unroll
-    for (int kk = 0; kk < T::kKK; ++kk) {
-      if (kk + 1 < T::kKK) {
-        read_frags((kk + 1) & 1, s, kk + 1);
-      } else if (s + 1 < n_my) {
-        // step s + 1 landed (steps up to s + kRing - 1 may still be in flight)
-        wait_steps<kPer, T::kRing - 2>(min(T::kRing - 2, n_my - 2 - s));
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of step s done
-        barrier();
-        read_frags(0, s + 1, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // keep those reads ahead of this sub-step's MFMAs
-      // On the last sub-step the freed slot's refill (step s + kRing) is issued one load
-      // after each MFMA, so the wave's load issue overlaps its own MFMAs.
-      const bool refill = kk + 1 == T::kKK && s + T::kRing < n_my;
-      constexpr int kMfma = T::kTM * T::kTN;
-#pragma unroll
-      for (int q = 0; q < (kMfma > kPer ? kMfma : kPer); ++q) {
-        if (q < kMfma) {
-          const int rb = q / T::kTN, cb = q % T::kTN;
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfg[kk & 1][cb], af[kk & 1][rb],
-                                                                acc[rb][cb], 0, 0, 0);
+      for (int kk = 0; kk < T::kKK; ++kk) {
+        if (kk + 1 < T::kKK) {
+          read_frags((kk + 1) & 1, s, kk + 1);
+        } else if (s + 1 < n_my) {
+          // step s + 1 landed (steps up to s + kRing - 1 may still be in flight)
+          wait_steps<kPer, T::kRing - 2>(min(T::kRing - 2, n_my - 2 - s));
+          __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of step s done
+          barrier();
+          read_frags(0, s + 1, 0);
         }
-        if (q < kPer && refill) issue_one(s + T::kRing, q);
-        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);  // keep those reads ahead of this sub-step's MFMAs
+        // On the last sub-step the freed slot's refill (step s + kRing) is issued one load
+        // after each MFMA, so the wave's load issue overlaps its own MFMAs.
+        const bool refill = kk + 1 == T::kKK && s + T::kRing < n_my;
+        constexpr int kMfma = T::kTM * T::kTN;
+#pragma unroll
+        for (int q = 0; q < (kMfma > kPer ? kMfma : kPer); ++q) {
+          if (q < kMfma) {
+            const int rb = q / T::kTN, cb = q % T::kTN;
+            acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfg[kk & 1][cb], af[kk & 1][rb],
+                                                                  acc[rb][cb], 0, 0, 0);
+          }
+          if (q < kPer && refill) issue_one(s + T::kRing, q);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
-  }
+  };
+  run_segments(segs, acc, steps);
 
-  tile_epilogue<T, kF32Out, kPartial, kArgmax, kAppend>(a, lds, acc, row0, col0, tn, sp, wm, wn, w,
-                                                        lane);
+  tile_epilogue<T, kF32Out, false, kArgmax, false>(a, lds, acc, row0, col0, tn, sp, wm, wn, w, lane);
 }
 
-// The 256 x 256 tile: one wave per SIMD, each 128 x 128.  A step is 64 k of both operands,
-// four 16 KiB halves (x rows 0-127 and 128-255: A0, A1; W rows likewise: B0, B1), double
-// buffered, and four phases of 32 MFMAs per wave, one per quadrant, in the order (A0,B0)
-// (A0,B1) (A1,B1) (A1,B0).
+// The large tiles: one wave per SIMD, each a quarter of the tile (128 x 128 of 256 x 256).  A
+// step is 64 k of both operands, four halves (x rows: A0, A1; W rows: B0, B1), kRing steps in
+// LDS, and four phases per wave, one per quadrant, in the order (A0,B0) (A0,B1) (A1,B1)
+// (A1,B0).
 //  * Every phase reads from LDS the half the next phase adds (B1, A1, A0(t+1), B0(t+1)), and
-//    issues the DMA of one half (A1(t+1), A0(t+2), B0(t+2), B1(t+2)), spread between its
-//    MFMAs, so no wait sits in front of an MFMA and a half has 3 phases or more to land.
-//  * Two barriers per step, each behind a vmcnt that leaves the newest three halves in
-//    flight: after phase 2 A0(t+1) and B0(t+1) are in LDS for every wave, after phase 4
-//    B1(t+1) and A1(t+1).  A half's slot is refilled only after a barrier that follows every
-//    wave's last use of it: fragments are consumed by MFMAs before the barrier, except
-//    A0(t+1)'s, which the lgkmcnt before the second barrier waits for (B0(t+1)'s 8 are
-//    newer; they are consumed in phase 1 of t+1, a barrier before B0's refill).
-//  * What bounds it: the MFMAs at the clock the card holds under them (taking all DMA out of
-//    the loop changes 289 us to 292 on 8192 x 6144 x 4096, all waits and barriers to 282),
-//    then ~5 us per tile to start and to store.  16 x 16 x 32 MFMAs beat 32 x 32 x 16 here
-//    (289 against 313 us): 16-cycle steps leave the wave's other instructions more places to
-//    issue.  128 x 128 per wave reads each fragment for 8 MFMAs, 128 KiB of LDS reads per
-//    step against 192 KiB for the 8-wave tile this replaces.
-//  * 8192 rows, qkv / o_proj / gate_up / down: 325 / 221 / 1285 / 604 us (8 waves, 32 x 32
-//    MFMAs, the next step staged in one burst) -> 284 / 192 / 1158 / 545 us, 1.42-1.51
-//    PFLOP/s; 2048 rows 94 / 77 / 330 / 181 -> 85 / 71 / 298 / 160 us.
-template <bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
-__global__ void __launch_bounds__(TileL::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
-  using T = TileL;
+//    issues the DMA of one half (A1(t+R-1), A0(t+R), B0(t+R), B1(t+R), R = kRing), spread
+//    between its MFMAs, so no wait sits in front of an MFMA and a half has 3 phases or more
+//    to land.
+//  * Two barriers per step, each behind a vmcnt that leaves the newest halves in flight:
+//    after phase 2 A0(t+1) and B0(t+1) are in LDS for every wave, after phase 4 B1(t+1) and
+//    A1(t+1).  A half's slot is refilled only after a barrier that follows every wave's last
+//    use of it: fragments are consumed by MFMAs before the barrier, except A0(t+1)'s, which
+//    the lgkmcnt before the second barrier waits for (B0(t+1)'s are newer; they are consumed
+//    in phase 1 of t+1, a barrier before B0's refill).
+//  * What bounds the 256 x 256 tile: the MFMAs at the clock the card holds under them (taking
+//    all DMA out of the loop changes 289 us to 292 on 8192 x 6144 x 4096, all waits and
+//    barriers to 282), then ~5 us per tile to start and to store.  16 x 16 x 32 MFMAs beat
+//    32 x 32 x 16 here (289 against 313 us): 16-cycle steps leave the wave's other
+//    instructions more places to issue.  128 x 128 per wave reads each fragment for 8 MFMAs.
+//  * 256 x 256, 8192 rows, qkv / o_proj / gate_up / down: 325 / 221 / 1285 / 604 us (8 waves,
+//    32 x 32 MFMAs, the next step staged in one burst) -> 284 / 192 / 1158 / 545 us,
+//    1.42-1.51 PFLOP/s.  256 x 128 and 128 x 128 against their 8- and 4-wave predecessors:
+//    qkv at 1000 rows 61 -> 52 us, o_proj at 700 rows 39 -> 33, gate_up at 512 rows (256 x
+//    256) 122 -> 94, down at 700 rows (256 x 256, K split 5 ways) 93 -> 74.
+template <class T, bool kNT, bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
+__global__ void __launch_bounds__(T::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
+  constexpr int kRing = T::kRing, kQM = T::kQM, kQN = T::kQN, dA = T::kDmaA, dB = T::kDmaB;
   __shared__ __attribute__((aligned(1024))) char lds[kGemmLds<T, kAppend>];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -467,66 +546,86 @@ __global__ void __launch_bounds__(TileL::kThreads, 1) gemm_quad_kernel(GemmArgs 
   const int n = (nst - sp + a.splits - 1) / a.splits;  // >= 1: splits <= steps
   const long long kstride = (long long)a.splits * T::kBK;
 
-  // LDS: x halves of buffer b at b * 32 KiB + half * 16 KiB, W halves 64 KiB further on.
-  // Wave w's DMA instruction i of a half covers rows 32 w + 8 i + lane / 8; a lane fills LDS
-  // chunk lane % 8 of its row, so it reads global chunk (lane % 8) ^ swz(row).
-  constexpr int kB = 4 * T::kHalf, kDma = 4;
-  uint32_t off_a[2][kDma], off_b[2][kDma];
+  // LDS: the x halves of slot b at b * 2 kHalfA, the W halves at kB + b * 2 kHalfB.
+  // Wave w's DMA instruction i of a half covers rows 8 (w d + i) + lane / 8 (d instructions
+  // per wave); a lane fills LDS chunk lane % 8 of its row, so it reads global chunk
+  // (lane % 8) ^ swz(row).
+  constexpr int kB = kRing * 2 * T::kHalfA;
+  uint32_t off_a[2][dA], off_b[2][dB];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) {
-      const int r = 32 * w + 8 * i + (lane >> 3);
-      const uint32_t c = ((lane & 7) ^ T::swz(r)) * 16;
-      const int gr = min(row0 + 128 * h + r, a.M - 1);
-      off_a[h][i] = (uint32_t)((long long)gr * a.ldx * 2) + c;
-      off_b[h][i] = (uint32_t)((long long)(col0 + 128 * h + r) * a.ldw * 2) + c;
+    for (int i = 0; i < dA; ++i) {
+      const int r = 8 * (w * dA + i) + (lane >> 3);
+      const int gr = min(row0 + T::kBM / 2 * h + r, a.M - 1);
+      off_a[h][i] = (uint32_t)((long long)gr * a.ldx * 2) + ((lane & 7) ^ T::swz(r)) * 16;
     }
-  const uint32_t dst0 = lds_base + w * (kDma * 1024);
-  auto stage_a = [&](const uint16_t* xs, int h, int buf, int i) {
-    dma16(xs, off_a[h][i], dst0 + (2 * buf + h) * T::kHalf + i * 1024);
+#pragma unroll
+    for (int i = 0; i < dB; ++i) {
+      const int r = 8 * (w * dB + i) + (lane >> 3);
+      off_b[h][i] = (uint32_t)((long long)(col0 + T::kBN / 2 * h + r) * a.ldw * 2) +
+                    ((lane & 7) ^ T::swz(r)) * 16;
+    }
+  }
+  const uint32_t dst_a = lds_base + w * (dA * 1024), dst_b = lds_base + kB + w * (dB * 1024);
+  auto stage_a = [&](const uint16_t* xs, int h, int slot, int i) {
+    dma16(xs, off_a[h][i], dst_a + (2 * slot + h) * T::kHalfA + i * 1024);
   };
-  auto stage_b = [&](const uint16_t* ws, int h, int buf, int i) {
-    dma16(ws, off_b[h][i], dst0 + kB + (2 * buf + h) * T::kHalf + i * 1024);
+  auto stage_b = [&](const uint16_t* ws, int h, int slot, int i) {
+    dma16_w<kNT>(ws, off_b[h][i], dst_b + (2 * slot + h) * T::kHalfB + i * 1024);
   };
-  // the k steps' pointers: step 0, 1 (xs1, ws1) and, in the loop, t + 2; past the end the
-  // last step is staged again (never read), so that every wait count holds
-  const uint16_t* xs0 = a.x + (long long)sp * T::kBK;
-  const uint16_t* ws0 = a.w + (long long)sp * T::kBK;
-  const uint16_t* xs1 = n > 1 ? xs0 + kstride : xs0;
-  const uint16_t* ws1 = n > 1 ? ws0 + kstride : ws0;
+  // xs, ws: where the newest staged step starts; past the end the last step is staged again
+  // (never read), so that every wait count holds.  xs_prev: the step before it.
+  const uint16_t* xs = a.x + (long long)sp * T::kBK;
+  const uint16_t* ws = a.w + (long long)sp * T::kBK;
+  // one row tile, unsplit, up to 128 rows: W streams from HBM
+  constexpr bool kSeg = kNT && T::kBM == 128;
+  const Segments segs{n, kSeg ? (int)(blockIdx.x >> 3) & 3 : 0};
+  int pos = segs.first();
+  xs += pos * kstride;
+  ws += pos * kstride;
+  auto advance = [&](bool more) {
+    if (!more) return;
+    const long long d = ++pos == n ? kstride - n * kstride : kstride;
+    pos = pos == n ? 0 : pos;
+    xs += d;
+    ws += d;
+  };
+  const uint16_t* xs_prev = xs;
 #pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_a(xs0, 0, 0, i);
+  for (int b = 0; b < kRing; ++b) {  // every slot but A1 of the last
 #pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_b(ws0, 0, 0, i);
+    for (int i = 0; i < dA; ++i) stage_a(xs, 0, b, i);
 #pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_b(ws0, 1, 0, i);
+    for (int i = 0; i < dB; ++i) stage_b(ws, 0, b, i);
 #pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_a(xs0, 1, 0, i);
+    for (int i = 0; i < dB; ++i) stage_b(ws, 1, b, i);
+    xs_prev = xs;
+    if (b + 1 < kRing) {
 #pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_a(xs1, 0, 1, i);
-#pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_b(ws1, 0, 1, i);
-#pragma unroll
-  for (int i = 0; i < kDma; ++i) stage_b(ws1, 1, 1, i);
+      for (int i = 0; i < dA; ++i) stage_a(xs, 1, b, i);
+      advance(b + 1 < n);
+    }
+  }
 
-  // fragment (r, kk) of a half: row 64 * wave + 16 r + lane % 16, 16-byte chunk 4 kk + lane / 16
+  // fragment (r, kk) of a half: row (wave's first) + 16 r + lane % 16, 16-byte chunk
+  // 4 kk + lane / 16
   int pa[2], pb[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     const int c = ((4 * kk + (lane >> 4)) ^ T::swz(lane & 15)) * 16;
-    pa[kk] = (wm * 64 + (lane & 15)) * T::kPitch + c;
-    pb[kk] = kB + (wn * 64 + (lane & 15)) * T::kPitch + c;
+    pa[kk] = (wm * (T::kBM / 4) + (lane & 15)) * T::kPitch + c;
+    pb[kk] = kB + (wn * (T::kBN / 4) + (lane & 15)) * T::kPitch + c;
   }
-  bf16x8 af[2][4][2], bf[2][4][2];  // [half][r][kk]
-  // fragment f = 4 kk + r of half h, in the buffer that pa / pb point at
+  bf16x8 af[2][kQM][2], bf[2][kQN][2];  // [half][r][kk]
+  // fragment f = kk * (blocks) + r of half h, in the slot that pa / pb point at
   auto read_a = [&](int h, int f) {
-    af[h][f & 3][f >> 2] = *reinterpret_cast<const bf16x8*>(lds + pa[f >> 2] + h * T::kHalf +
-                                                            (f & 3) * 16 * T::kPitch);
+    af[h][f % kQM][f / kQM] = *reinterpret_cast<const bf16x8*>(
+        lds + pa[f / kQM] + h * T::kHalfA + (f % kQM) * 16 * T::kPitch);
   };
   auto read_b = [&](int h, int f) {
-    bf[h][f & 3][f >> 2] = *reinterpret_cast<const bf16x8*>(lds + pb[f >> 2] + h * T::kHalf +
-                                                            (f & 3) * 16 * T::kPitch);
+    bf[h][f % kQN][f / kQN] = *reinterpret_cast<const bf16x8*>(
+        lds + pb[f / kQN] + h * T::kHalfB + (f % kQN) * 16 * T::kPitch);
   };
   float4_t acc[T::kTM][T::kTN];
 #pragma unroll
@@ -534,61 +633,84 @@ __global__ void __launch_bounds__(TileL::kThreads, 1) gemm_quad_kernel(GemmArgs 
 #pragma unroll
     for (int cb = 0; cb < T::kTN; ++cb) acc[rb][cb] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  // One phase: the 32 MFMAs of quadrant (x half i, W half j), kk outermost; between(g) places
-  // fragment reads and DMA instructions after each pair g.
+  // One phase: the MFMAs of quadrant (x half i, W half j), kk outermost; between(q) places
+  // fragment reads and DMA instructions after MFMA q.
+  constexpr int kN = 2 * kQM * kQN;
   auto phase = [&](int i, int j, auto&& between) {
 #pragma unroll
-    for (int q = 0; q < 32; ++q) {
-      const int kk = q >> 4, r = (q >> 2) & 3, c = q & 3;
-      acc[4 * i + r][4 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          bf[j][c][kk], af[i][r][kk], acc[4 * i + r][4 * j + c], 0, 0, 0);
-      if (q & 1) between(q >> 1);
+    for (int q = 0; q < kN; ++q) {
+      const int kk = q / (kQM * kQN), r = q / kQN % kQM, c = q % kQN;
+      acc[kQM * i + r][kQN * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          bf[j][c][kk], af[i][r][kk], acc[kQM * i + r][kQN * j + c], 0, 0, 0);
+      between(q);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  wait_vm<3 * kDma>();  // step 0
+  // after MFMA q: those of `count` reads spread over the phase's first half, of `count` DMA
+  // instructions spread over all of it
+  auto reads = [&](int q, int count, auto&& f) {
+#pragma unroll
+    for (int e = 0; e < count; ++e)
+      if (((2 * e + 1) * (kN / 2)) / (2 * count) == q) f(e);
+  };
+  auto stages = [&](int q, int count, auto&& f) {
+#pragma unroll
+    for (int e = 0; e < count; ++e)
+      if (((2 * e + 1) * kN) / (2 * count) == q) f(e);
+  };
+  wait_vm<2 * dB + dA + (kRing - 2) * 2 * (dA + dB)>();  // step 0
   barrier();
 #pragma unroll
-  for (int f = 0; f < 8; ++f) read_a(0, f);
+  for (int f = 0; f < 2 * kQM; ++f) read_a(0, f);
 #pragma unroll
-  for (int f = 0; f < 8; ++f) read_b(0, f);
-  for (int t = 0; t < n; ++t) {
-    const int buf = t & 1;
-    const bool more = t + 2 < n;
-    const uint16_t* xs2 = more ? xs1 + kstride : xs1;
-    const uint16_t* ws2 = more ? ws1 + kstride : ws1;
-    phase(0, 0, [&](int g) {
-      if (g < 8) read_b(1, g);
-      if ((g & 3) == 1) stage_a(xs1, 1, buf ^ 1, g >> 2);
-    });
-    phase(0, 1, [&](int g) {
-      if (g < 8) read_a(1, g);
-      if ((g & 3) == 1) stage_a(xs2, 0, buf, g >> 2);
-    });
-    wait_vm<3 * kDma>();  // A0(t+1), B0(t+1)
-    barrier();
+  for (int f = 0; f < 2 * kQN; ++f) read_b(0, f);
+  int cur = 0;  // step t's slot
+  int t = 0;
+  auto steps = [&](int end) {
+    for (; t < end; ++t) {
+      const int prev = cur == 0 ? kRing - 1 : cur - 1;
+      const bool more = t + kRing < n;
+      advance(more);
+      phase(0, 0, [&](int q) {
+        reads(q, 2 * kQN, [&](int f) { read_b(1, f); });
+        stages(q, dA, [&](int i) { stage_a(xs_prev, 1, prev, i); });  // A1(t + kRing - 1)
+      });
+      phase(0, 1, [&](int q) {
+        reads(q, 2 * kQM, [&](int f) { read_a(1, f); });
+        stages(q, dA, [&](int i) { stage_a(xs, 0, cur, i); });  // A0(t + kRing)
+      });
+      wait_vm<dB + 2 * dA + (kRing - 2) * 2 * (dA + dB)>();  // A0(t+1), B0(t+1)
+      barrier();
+      const int dslot = cur == kRing - 1 ? 1 - kRing : 1;  // to step t + 1's slot
+      const int da = dslot * 2 * T::kHalfA, db = dslot * 2 * T::kHalfB;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {  // the other buffer
-      pa[kk] ^= 2 * T::kHalf;
-      pb[kk] ^= 2 * T::kHalf;
+      for (int kk = 0; kk < 2; ++kk) {
+        pa[kk] += da;
+        pb[kk] += db;
+      }
+      phase(1, 1, [&](int q) {
+        reads(q, 2 * kQM, [&](int f) { read_a(0, f); });
+        stages(q, dB, [&](int i) { stage_b(ws, 0, cur, i); });  // B0(t + kRing)
+      });
+      phase(1, 0, [&](int q) {  // B0(t+1)'s fragments as B0(t)'s are used up
+        if (q >= kN / 2 && q < kN / 2 + kQN) read_b(0, q - kN / 2);
+        if (q == kN - 1)
+#pragma unroll
+          for (int f = kQN; f < 2 * kQN; ++f) read_b(0, f);
+        stages(q, dB, [&](int i) { stage_b(ws, 1, cur, i); });  // B1(t + kRing)
+      });
+      wait_vm<2 * dB + dA + (kRing - 2) * 2 * (dA + dB)>();  // B1(t+1), A1(t+1)
+      // lgkmcnt(2 kQN): A0(t+1) is read (B0's are newer)
+      __builtin_amdgcn_s_waitcnt(0xC07F | (2 * kQN) << 8);
+      barrier();
+      xs_prev = xs;
+      cur = cur == kRing - 1 ? 0 : cur + 1;
     }
-    phase(1, 1, [&](int g) {
-      if (g < 8) read_a(0, g);
-      if ((g & 3) == 1) stage_b(ws2, 0, buf, g >> 2);
-    });
-    phase(1, 0, [&](int g) {  // B0(t+1)'s fragments as B0(t)'s are used up
-      if (g >= 8 && g < 12) read_b(0, g - 8);
-      if (g == 15)
-#pragma unroll
-        for (int f = 4; f < 8; ++f) read_b(0, f);
-      if ((g & 3) == 1) stage_b(ws2, 1, buf, g >> 2);
-    });
-    wait_vm<3 * kDma>();  // B1(t+1), A1(t+1)
-    __builtin_amdgcn_s_waitcnt(0xC87F);  // lgkmcnt(8): A0(t+1) is read
-    barrier();
-    xs1 = xs2;
-    ws1 = ws2;
-  }
+  };
+  if constexpr (kSeg)
+    run_segments(segs, acc, steps);
+  else
+    steps(n);
   wait_vm<0>();  // the DMAs past the end: the LDS is reused or given back
 
   // the epilogue's addresses are computed after the loop, not held in registers through it
@@ -596,12 +718,204 @@ __global__ void __launch_bounds__(TileL::kThreads, 1) gemm_quad_kernel(GemmArgs 
   asm volatile("" : "+v"(elane), "+s"(erow0), "+s"(ecol0));
   // ... and the accumulators stay in AGPRs up to here (VALU ops cannot read those: without
   // this the allocator spreads the epilogue's copies into the loop and spills)
+  if constexpr (T::kTM * T::kTN >= 64) {
 #pragma unroll
-  for (int rb = 0; rb < T::kTM; ++rb)
+    for (int rb = 0; rb < T::kTM; ++rb)
 #pragma unroll
-    for (int cb = 0; cb < T::kTN; ++cb) asm volatile("" : "+a"(acc[rb][cb]));
+      for (int cb = 0; cb < T::kTN; ++cb) asm volatile("" : "+a"(acc[rb][cb]));
+  }
   tile_epilogue<T, kF32Out, kPartial, kArgmax, kAppend>(a, lds, acc, erow0, ecol0, tn, sp, wm, wn, w,
                                                         elane);
+}
+
+// A few rows: no K split over workgroups and no reduction launch.  A workgroup takes a tile of
+// kBM x kBN outputs over the whole of K, each of its waves a contiguous part of the k steps,
+// staged through a ring of kSlots steps in LDS of the wave's own, so the loop has no barrier;
+// the waves' fp32 sums meet in LDS at the end, added in wave order.  Tiles are small enough
+// that one round of workgroups covers the CUs (o_proj at 6 rows: 8 x 16).
+//  * A step's blocks of 16 rows are consumed as they land: block b is read, block b - 1's LDS
+//    is refilled with its rows of step t + kSlots and (x blocks) its MFMAs issue, so nearly
+//    the whole ring stays in flight.
+//  * What bounds it: HBM for W and the launch at a few rows (o_proj at 6 rows 9.1 us against
+//    7.4 for its W stream alone), the rate at which a CU stages x from L2 above (~70 KB/us).
+//  * W cold, against the K-split tiles and their reduction: o_proj at 6 / 32 / 100 / 250 rows
+//    14.1 / 14.7 / 18.5 / 23.3 -> 8.9 / 10.6 / 14.7 / 19.4 us, qkv at 6 / 32 / 100 rows 15.6 /
+//    16.2 / 19.7 -> 11.2 / 12.8 / 17.6, down at 6 / 64 rows 27.3 / 32.1 -> 21.0 / 27.3.
+template <int kXB8_, int kWB8_, int kWaves_>
+struct Slab {
+  static constexpr int kXB8 = kXB8_, kWB8 = kWB8_, kWaves = kWaves_, kThreads = 64 * kWaves_;
+  static constexpr int kBM = 8 * kXB8, kBN = 8 * kWB8;  // both staged 8 rows per DMA
+  static constexpr int kMB = (kXB8 + 1) / 2, kNB = (kWB8 + 1) / 2;  // 16 x 16 blocks
+  static constexpr int kSlot = (kBM + kBN) * 128;      // one step: 64 k of every row
+  // an odd kXB8's last block reads 8 rows past the slot (never stored): 1 KiB more
+  static constexpr int kPad = kXB8 % 2 * 1024;
+  static constexpr int kFit = (160 * 1024 - kPad) / kWaves / kSlot;
+  static constexpr int kDma = kXB8 + kWB8;
+  static constexpr int kMost = 60 / kDma < 6 ? 60 / kDma : 6;  // vmcnt counts to 63
+  static constexpr int kSlots = kFit < kMost ? kFit : kMost;
+  // DMA instructions (8 rows each) of block b of a step: 16 W rows (b < kNB), then 16 x rows
+  __host__ __device__ static constexpr int dmas(int b) {
+    return (b < kNB ? 2 * b + 2 <= kWB8 : 2 * (b - kNB) + 2 <= kXB8) ? 2 : 1;
+  }
+  static constexpr int kRed = kWaves * kMB * kNB * 1024;  // the waves' sums
+  static constexpr int kRingBytes = kWaves * kSlots * kSlot + kPad;
+  static constexpr int kLds = kRingBytes > kRed ? kRingBytes : kRed;
+  static_assert(kSlots >= 2 && kLds <= 160 * 1024 && kSlots * kDma < 64, "ring");
+};
+
+// f(integral_constant<int, b>) for every block of a step, unrolled.
+template <class T, int b = 0, class F>
+__device__ __forceinline__ void slab_blocks(F&& f) {
+  if constexpr (b < T::kNB + T::kMB) {
+    f(std::integral_constant<int, b>{});
+    slab_blocks<T, b + 1>(f);
+  }
+}
+
+template <class T, bool kF32Out, bool kPartial>
+__global__ void __launch_bounds__(T::kThreads, 1) gemm_slab_kernel(GemmArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[T::kLds];
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tm, tn, sp;
+  tile_of(a, tm, tn, sp);
+  const int row0 = tm * T::kBM, col0 = tn * T::kBN;
+  // the wave's k steps: part w of the workgroup's part sp
+  const int nst = a.K / 64, parts = T::kWaves * a.splits, part = sp * T::kWaves + w;
+  const int s0 = part * nst / parts, n = (part + 1) * nst / parts - s0;
+  auto swz = [](int r) { return (r >> 1) & 7; };
+  // slot: W rows, then x rows, 128 bytes each, chunk c of row r at c ^ swz(r)
+  uint32_t off_w[T::kWB8], off_x[T::kXB8];
+#pragma unroll
+  for (int i = 0; i < T::kWB8; ++i) {
+    const int r = 8 * i + (lane >> 3);
+    off_w[i] = (uint32_t)((long long)(col0 + r) * a.ldw * 2) + ((lane & 7) ^ swz(r)) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < T::kXB8; ++i) {
+    const int r = 8 * i + (lane >> 3);
+    off_x[i] = (uint32_t)((long long)min(row0 + r, a.M - 1) * a.ldx * 2) + ((lane & 7) ^ swz(r)) * 16;
+  }
+  float4_t acc[T::kMB][T::kNB];
+#pragma unroll
+  for (int rb = 0; rb < T::kMB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < T::kNB; ++cb) acc[rb][cb] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const uint32_t ring = w * (T::kSlots * T::kSlot);
+  int pw[2];  // fragment kk of block b: row 16 b + lane % 16, chunk 4 kk + lane / 16
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+    pw[kk] = ring + (lane & 15) * 128 + ((4 * kk + (lane >> 4)) ^ swz(lane & 15)) * 16;
+  if (n > 0) {
+    const uint16_t* xs = a.x + (long long)s0 * 64;
+    const uint16_t* ws = a.w + (long long)s0 * 64;
+    int left = n - 1;  // steps after the one that xs and ws point at
+    constexpr int kBlocks = T::kNB + T::kMB;
+    auto stage = [&](int slot, int b) {
+      const uint32_t dst = lds_base + ring + slot * T::kSlot;
+#pragma unroll
+      for (int i = 0; i < T::dmas(b); ++i) {
+        const int q = b < T::kNB ? 2 * b + i : 2 * (b - T::kNB) + i;
+        if (b < T::kNB) {
+          dma16(ws, off_w[q], dst + q * 1024);
+        } else {
+          dma16(xs, off_x[q], dst + (T::kWB8 + q) * 1024);
+        }
+      }
+    };
+    // the next step; past the end the last one is staged again (never read), so that every
+    // wait count holds
+    auto advance = [&]() {
+      const int d = left > 0 ? 64 : 0;
+      --left;
+      xs += d;
+      ws += d;
+    };
+#pragma unroll
+    for (int k = 0; k < T::kSlots; ++k) {
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) stage(k, b);
+      advance();
+    }
+    int slot = 0;
+    for (int t = 0; t < n; ++t) {
+      const char* sb = lds + slot * T::kSlot;
+      bf16x8 wf[T::kNB][2], xf[2][2];
+      // block b: its fragments in registers, so its LDS is refilled; an x block's MFMAs
+      auto finish = [&](int b) {
+        asm volatile("" ::: "memory");
+        stage(slot, b);
+        if (b >= T::kNB) {
+          const int rb = b - T::kNB;
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int cb = 0; cb < T::kNB; ++cb)
+              acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[cb][kk], xf[rb & 1][kk],
+                                                                    acc[rb][cb], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      constexpr int kAll = T::kSlots * T::kDma;
+      auto read = [&](int b, auto wait_tag) {
+        // block b's DMAs have landed: newer are the rest of the ring and the blocks of step
+        // t + kSlots staged so far (up to b - 2)
+        wait_vm<decltype(wait_tag)::value>();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          if (b < T::kNB)
+            wf[b][kk] = *reinterpret_cast<const bf16x8*>(sb + pw[kk] + b * 2048);
+          else
+            xf[(b - T::kNB) & 1][kk] = *reinterpret_cast<const bf16x8*>(
+                sb + pw[kk] + T::kWB8 * 1024 + (b - T::kNB) * 2048);
+        }
+      };
+      slab_blocks<T>([&](auto tag) {
+        constexpr int b = decltype(tag)::value;
+        constexpr int d0 = T::dmas(b), d1 = b > 0 ? T::dmas(b > 0 ? b - 1 : 0) : 0;
+        read(b, std::integral_constant<int, kAll - d0 - d1>{});
+        if constexpr (b > 0) {
+          __builtin_amdgcn_s_waitcnt(0xC27F);  // lgkmcnt(2): block b - 1's fragments
+          finish(b - 1);
+        }
+      });
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      finish(kBlocks - 1);
+      advance();
+      slot = slot + 1 == T::kSlots ? 0 : slot + 1;
+    }
+  }
+  wait_vm<0>();  // every DMA has landed: the LDS is reused
+  __syncthreads();
+#pragma unroll
+  for (int rb = 0; rb < T::kMB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < T::kNB; ++cb)
+      *reinterpret_cast<float4_t*>(lds + ((w * T::kMB + rb) * T::kNB + cb) * 1024 + lane * 16) =
+          acc[rb][cb];
+  __syncthreads();
+  // thread -> (row, 4 columns), consecutive threads along a row
+  constexpr int kRow4 = T::kBN / 4;
+  for (int e = threadIdx.x; e < T::kBM * kRow4; e += T::kThreads) {
+    const int r = e / kRow4, c = e % kRow4 * 4;
+    const int m = row0 + r;
+    if (m >= a.M) break;
+    const char* src = lds + ((r >> 4) * T::kNB + (c >> 4)) * 1024 + ((r & 15) + ((c & 15) >> 2) * 16) * 16;
+    float4_t v = *reinterpret_cast<const float4_t*>(src);
+#pragma unroll
+    for (int k = 1; k < T::kWaves; ++k)
+      v += *reinterpret_cast<const float4_t*>(src + k * T::kMB * T::kNB * 1024);
+    const int nc = col0 + c;
+    if (kPartial)
+      *reinterpret_cast<float4_t*>(a.part + ((long long)sp * a.M + m) * a.N + nc) = v;
+    else if (kF32Out)
+      *reinterpret_cast<float4_t*>(static_cast<float*>(a.y) + m * a.ldy + nc) = v;
+    else
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + m * a.ldy + nc) =
+          make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+  }
 }
 
 // The QKV projection's epilogue fused with the per-head norm + RoPE + paged append
@@ -813,65 +1127,171 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(GemmArgs a) {
   }
 }
 
-// The launch plan of one call: up to 128 rows the tile with the fewest rows that covers
-// M (tile 1, 2, 3 = 128, 64, 32 rows by 128 columns); up to 1024 rows 256 x 128 (tile 4);
-// above, 256 x 256 (tile 0) when N allows.  When the tiles alone leave CUs idle, K is
-// split so that tiles x splits fill the 256 CUs once (the kernels run one workgroup per
-// CU).
-struct GemmPlan {
-  int tile, bm, bn, splits, m_tiles, n_tiles;
-};
-GemmPlan gemm_plan(int M, int N, int K) {
-  GemmPlan p;
-  p.tile = M > 1024 && N % 256 == 0 ? 0 : M > 128 ? 4 : M > 64 ? 1 : M > 32 ? 2 : 3;
-  // 129..256 rows over few columns (o_proj, down: 32 tiles of 256 x 128, split 8 ways):
-  // two 128-row tiles halve the split count and the partial traffic (measured 23.0 ->
-  // 21.2 us on o_proj at 256 rows; with 48 or more tiles the 256-row tile wins)
-  if (M > 128 && M <= 256 && N / 128 < 40) p.tile = 1;
-  p.bm = p.tile == 0 || p.tile == 4 ? 256 : p.tile == 1 ? 128 : p.tile == 2 ? 64 : 32;
-  p.bn = p.tile == 0 ? 256 : 128;
-  p.m_tiles = (M + p.bm - 1) / p.bm;
-  p.n_tiles = N / p.bn;
-  const int tiles = p.m_tiles * p.n_tiles;
-  const int nst = K / kGK;
-  int s = tiles >= 160 ? 1 : 256 / tiles;
-  if (s > 16) s = 16;
-  if (s > nst) s = nst;
-  p.splits = s < 1 ? 1 : s;
-  return p;
-}
-
 bool gemm_shape_ok(int M, int N, int K) {
   return M >= 0 && N > 0 && K > 0 && N % 128 == 0 && K % kGK == 0;
 }
 
-template <class T>
-void launch_argmax(const GemmArgs& a, hipStream_t st) {
-  if constexpr (std::is_same_v<T, TileL>) {
-    hipLaunchKernelGGL((gemm_quad_kernel<false, false, true>),
-                       dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
-    return;
-  } else
-  hipLaunchKernelGGL((gemm_kernel<T, false, false, true>),
-                     dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
+// K splits that fqa_gemm_workspace_bytes has room for at least (a fixed rule, so that a
+// workspace sized once stays valid): as many as bring tiles of 32, 64, 128 or 256 rows (the
+// fewest that cover M, 256 above) by 128 columns (256 above 1024 rows) to the 256 CUs once,
+// at most 16, one where 160 tiles or more exist.
+int sized_splits(int M, int N, int K) {
+  int bm = M > 128 ? 256 : M > 64 ? 128 : M > 32 ? 64 : 32;
+  const int bn = M > 1024 && N % 256 == 0 ? 256 : 128;
+  if (M > 128 && M <= 256 && N / 128 < 40) bm = 128;
+  const int tiles = ((M + bm - 1) / bm) * (N / bn);
+  int s = tiles >= 160 ? 1 : 256 / tiles;
+  if (s > 16) s = 16;
+  if (s > K / kGK) s = K / kGK;
+  return s < 1 ? 1 : s;
+}
+
+// The slab tiles: {rows, columns} and, in slab_dispatch, their waves.
+constexpr int kSlabs[][2] = {{8, 16},  {8, 24},  {16, 16}, {16, 24}, {32, 16}, {32, 24}, {32, 32},
+                             {64, 32}, {64, 48}, {96, 32}, {96, 48}, {64, 64}, {96, 64}, {64, 96}};
+template <class F>
+bool slab_dispatch(int i, F&& f) {
+  switch (i) {
+    case 0: return f(Slab<1, 2, 8>{});
+    case 1: return f(Slab<1, 3, 8>{});
+    case 2: return f(Slab<2, 2, 8>{});
+    case 3: return f(Slab<2, 3, 8>{});
+    case 4: return f(Slab<4, 2, 4>{});
+    case 5: return f(Slab<4, 3, 4>{});
+    case 6: return f(Slab<4, 4, 4>{});
+    case 7: return f(Slab<8, 4, 4>{});
+    case 8: return f(Slab<8, 6, 4>{});
+    case 9: return f(Slab<12, 4, 4>{});
+    case 10: return f(Slab<12, 6, 4>{});
+    case 11: return f(Slab<8, 8, 4>{});
+    case 12: return f(Slab<12, 8, 4>{});
+    default: return f(Slab<8, 12, 4>{});
+  }
+}
+
+// The launch plan of one call.
+enum Tiles { kTileT, kTileS, kTileM, kTileH, kTileL, kSlab0 };
+struct GemmPlan {
+  int tile;  // Tiles; kSlab0 + i: kSlabs[i]
+  int bm, bn, splits, m_tiles, n_tiles;
+};
+
+// Chosen by a model of the time in us, fitted to measurements on 6144 x 4096, 4096 x 4096,
+// 24576 x 4096 and 4096 x 12288 at 6 to 2048 rows with W cold (within ~15% of each, and
+// nearly always the measured order):
+//  * Tiles of 128 columns or more: 2.4 for the launch and, per round of 256 workgroups, 5 to
+//    start and store and 1.29 (256 x 256), 0.78 (256 x 128) or 0.45 (128 x 128; 0.75 with a
+//    single row tile, whose W comes from HBM) per step of 64 k.
+//  * Slabs: 6, 1 per 70 KB that a workgroup stages and 1 per 4096 outputs of the tile (the
+//    sum over its waves); one round of workgroups; for x that fits an XCD's L2
+//    beside the W stream (3.5 MB: at 12288 k and 160 rows the slabs lose).
+//  * A K split adds the reduction: 2.5, 1 per split and 1 per million fp32 partials (8 MB).
+// Up to 128 rows with 160 column tiles or more (gate_up, lm_head) the smallest tile that
+// covers M streams W once at HBM's rate, and nothing is split.
+// max_splits bounds K splits; 1 (fqa_gemm_argmax, and shapes whose workspace is empty) also
+// leaves the slabs out, so that equal shapes sum in the same order.
+GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
+  const int nst = K / kGK;
+  auto make = [&](int tile, int bm, int bn, int s) {
+    return GemmPlan{tile, bm, bn, s, (M + bm - 1) / bm, N / bn};
+  };
+  if (M <= 128 && N / 128 >= 160)
+    return M > 64 ? make(kTileM, 128, 128, 1) : M > 32 ? make(kTileS, 64, 128, 1) : make(kTileT, 32, 128, 1);
+  GemmPlan best{};
+  float best_us = 3.4e38f;
+  auto consider = [&](const GemmPlan& p, float us) {
+    if (p.splits > 1) us += 2.5f + p.splits + 1e-6f * p.splits * M * N;
+    if (us < best_us) {
+      best_us = us;
+      best = p;
+    }
+  };
+  const int quads[3][3] = {{kTileL, 256, 256}, {kTileH, 256, 128}, {kTileM, 128, 128}};
+  for (const auto& q : quads) {
+    if (N % q[2]) continue;
+    for (int s = 1; s <= max_splits && s <= 16 && s <= nst; ++s) {
+      const GemmPlan p = make(q[0], q[1], q[2], s);
+      const long long g = (long long)p.m_tiles * p.n_tiles * s;
+      if (s > 1 && g > 256) break;
+      const float step = q[0] == kTileL ? 1.29f : q[0] == kTileH ? 0.78f : p.m_tiles == 1 ? 0.75f : 0.45f;
+      consider(p, 2.4f + (float)((g + 255) / 256) * ((float)((nst + s - 1) / s) * step + 5.f));
+    }
+  }
+  if (max_splits > 1 && (long long)M * K * 2 <= 3500000) {
+    for (int i = 0; i < (int)(sizeof(kSlabs) / sizeof(kSlabs[0])); ++i) {
+      const int bm = kSlabs[i][0], bn = kSlabs[i][1];
+      if (N % bn) continue;
+      for (int s = 1; s <= 4 && s <= max_splits && s <= nst; s *= 2) {
+        const GemmPlan p = make(kSlab0 + i, bm, bn, s);
+        if ((long long)p.m_tiles * p.n_tiles * s > 256) break;
+        consider(p, 6.f + (bm + bn) * 2.f * K / s / 70e3f + bm * bn / 4096.f);
+      }
+    }
+  }
+  return best;
+}
+
+// The largest K split a call may use: what the shape's workspace is sized for, and beyond
+// that (not for the QKV width, whose size is fixed by sized_splits) what the plan would take
+// if `bytes` has room.
+int splits_allowed(int M, int N, int K, int64_t bytes) {
+  const int s = sized_splits(M, N, K);
+  if (s == 1 || N == kQkvStride) return s;
+  const int64_t fit = bytes / ((int64_t)M * N * 4);
+  return fit > 16 ? 16 : fit > s ? (int)fit : s;
+}
+
+template <class T, bool kNT>
+void launch_quad(const GemmArgs& a, bool f32, dim3 grid, hipStream_t st) {
+  if (f32)
+    hipLaunchKernelGGL((gemm_quad_kernel<T, kNT, true, false>), grid, dim3(T::kThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((gemm_quad_kernel<T, kNT, false, false>), grid, dim3(T::kThreads), 0, st, a);
 }
 template <class T>
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t st) {
   const dim3 grid((unsigned)(a.m_tiles * a.n_tiles * a.splits));
   const dim3 block(T::kThreads);
-  if constexpr (std::is_same_v<T, TileL>) {
+  if constexpr (kIsQuad<T>) {
     if (a.splits > 1)
-      hipLaunchKernelGGL((gemm_quad_kernel<false, true>), grid, block, 0, st, a);
-    else if (f32)
-      hipLaunchKernelGGL((gemm_quad_kernel<true, false>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, true>), grid, block, 0, st, a);
+    else if (T::kBN == 128 && a.m_tiles == 1)
+      launch_quad<T, T::kBN == 128>(a, f32, grid, st);
     else
-      hipLaunchKernelGGL((gemm_quad_kernel<false, false>), grid, block, 0, st, a);
-  } else if (a.splits > 1)
+      launch_quad<T, false>(a, f32, grid, st);
+  } else if (f32) {
+    hipLaunchKernelGGL((gemm_kernel<T, true>), grid, block, 0, st, a);
+  } else {
+    hipLaunchKernelGGL((gemm_kernel<T, false>), grid, block, 0, st, a);
+  }
+}
+template <class T>
+void launch_argmax(const GemmArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(a.m_tiles * a.n_tiles));
+  const dim3 block(T::kThreads);
+  if constexpr (!kIsQuad<T>)
     hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, block, 0, st, a);
-  else if (f32)
-    hipLaunchKernelGGL((gemm_kernel<T, true, false>), grid, block, 0, st, a);
+  else if (T::kBN == 128 && a.m_tiles == 1)
+    hipLaunchKernelGGL((gemm_quad_kernel<T, T::kBN == 128, false, false, true>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((gemm_kernel<T, false, false>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, false, true>), grid, block, 0, st, a);
+}
+template <class T>
+void launch_append(const GemmArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, false, false, true>),
+                     dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
+}
+// A slab's launch; planes: fp32 into a.part also without a split.
+template <class T>
+void launch_slab(const GemmArgs& a, bool f32, bool planes, hipStream_t st) {
+  const dim3 grid((unsigned)(a.m_tiles * a.n_tiles * a.splits));
+  const dim3 block(T::kThreads);
+  if (planes)
+    hipLaunchKernelGGL((gemm_slab_kernel<T, false, true>), grid, block, 0, st, a);
+  else if (f32)
+    hipLaunchKernelGGL((gemm_slab_kernel<T, true, false>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((gemm_slab_kernel<T, false, false>), grid, block, 0, st, a);
 }
 }  // namespace
 }  // namespace fqa
@@ -880,8 +1300,11 @@ using namespace fqa;
 
 extern "C" int64_t fqa_gemm_workspace_bytes(int32_t M, int32_t N, int32_t K) {
   if (!gemm_shape_ok(M, N, K) || M == 0) return 0;
-  const GemmPlan p = gemm_plan(M, N, K);
-  return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
+  const int sized = sized_splits(M, N, K);
+  if (sized == 1) return 0;
+  const int most = splits_allowed(M, N, K, INT64_MAX);
+  const int want = gemm_plan(M, N, K, most).splits;
+  return (int64_t)(want > sized ? want : sized) * M * N * 4;
 }
 
 namespace fqa {
@@ -899,50 +1322,56 @@ static int gemm_prepare(const void* x, int64_t ldx, const void* w, int64_t ldw, 
   // DMA lane offsets are 32-bit: every row start of x and W must lie within 4 GiB
   if ((int64_t)(M - 1) * ldx * 2 >= (int64_t)1 << 32 || (int64_t)(N - 1) * ldw * 2 >= (int64_t)1 << 32)
     return FQA_EUNSUPPORTED;
-  p = gemm_plan(M, N, K);
+  const int sized = sized_splits(M, N, K);
+  if (sized > 1 && (!workspace || workspace_bytes < (int64_t)sized * M * N * 4 ||
+                    ((uintptr_t)workspace & 15)))
+    return FQA_EINVAL;
+  p = gemm_plan(M, N, K, splits_allowed(M, N, K, workspace_bytes));
   if ((int64_t)p.m_tiles * p.n_tiles * p.splits > 0x7fffffff) return FQA_EINVAL;
   a = GemmArgs{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), y, nullptr,
                ldx, ldw, ldy, M, N, K, p.splits, p.m_tiles, p.n_tiles};
-  if (p.splits > 1) {
-    if (!workspace || workspace_bytes < (int64_t)p.splits * M * N * 4 || ((uintptr_t)workspace & 15))
-      return FQA_EINVAL;
-    a.part = static_cast<float*>(workspace);
-  }
+  if (sized > 1) a.part = static_cast<float*>(workspace);
   return FQA_OK;
 }
 
-static void gemm_launch_main(const GemmArgs& a, const GemmPlan& p, bool f32, hipStream_t st) {
+// planes: a slab leaves fp32 in a.part also without a split
+static void gemm_launch_main(const GemmArgs& a, const GemmPlan& p, bool f32, bool planes,
+                             hipStream_t st) {
   switch (p.tile) {
-    case 0: launch_gemm<TileL>(a, f32, st); break;
-    case 4: launch_gemm<TileL8>(a, f32, st); break;
-    case 1: launch_gemm<TileM>(a, f32, st); break;
-    case 2: launch_gemm<TileS>(a, f32, st); break;
-    default: launch_gemm<TileT>(a, f32, st); break;
+    case kTileL: launch_gemm<TileL>(a, f32, st); break;
+    case kTileH: launch_gemm<TileH>(a, f32, st); break;
+    case kTileM: launch_gemm<TileM>(a, f32, st); break;
+    case kTileS: launch_gemm<TileS>(a, f32, st); break;
+    case kTileT: launch_gemm<TileT>(a, f32, st); break;
+    default:
+      slab_dispatch(p.tile - kSlab0, [&](auto t) {
+        launch_slab<decltype(t)>(a, f32, planes || a.splits > 1, st);
+        return true;
+      });
   }
 }
 
 int gemm_launch_partials(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
                          int64_t ldy, int32_t M, int32_t N, int32_t K, void* workspace,
-                         int64_t workspace_bytes, hipStream_t st, const GemmAppend* app,
+                         int64_t workspace_bytes, hipStream_t st, const GemmAppend& app,
                          bool* appended) {
   GemmArgs a;
   GemmPlan p;
-  if (appended) *appended = false;
+  *appended = false;
   const int rc = gemm_prepare(x, ldx, w, ldw, y, ldy, M, N, K, workspace, workspace_bytes, a, p);
   if (rc != FQA_OK || M == 0) return rc;
-  if (app && p.splits == 1 && N == kQkvStride && (p.tile == 0 || p.tile == 4)) {
-    a.app = *app;
-    const dim3 grid((unsigned)(a.m_tiles * a.n_tiles));
-    if (p.tile == 0)
-      hipLaunchKernelGGL((gemm_quad_kernel<false, false, false, true>), grid,
-                         dim3(TileL::kThreads), 0, st, a);
+  if (p.splits == 1 && p.tile < kSlab0) {  // (48 column tiles: never a 32- or 64-row tile)
+    a.app = app;
+    if (p.tile == kTileL)
+      launch_append<TileL>(a, st);
+    else if (p.tile == kTileH)
+      launch_append<TileH>(a, st);
     else
-      hipLaunchKernelGGL((gemm_kernel<TileL8, false, false, false, true>), grid,
-                         dim3(TileL8::kThreads), 0, st, a);
-    if (appended) *appended = true;
-    return 1;
+      launch_append<TileM>(a, st);
+    *appended = true;
+    return 0;
   }
-  gemm_launch_main(a, p, false, st);
+  gemm_launch_main(a, p, false, true, st);
   return p.splits;
 }
 
@@ -956,7 +1385,7 @@ extern "C" int fqa_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, 
   const int rc = gemm_prepare(x, ldx, w, ldw, y, ldy, M, N, K, workspace, workspace_bytes, a, p);
   if (rc != FQA_OK || M == 0) return rc;
   hipStream_t st = (hipStream_t)stream;
-  gemm_launch_main(a, p, y_f32 != 0, st);
+  gemm_launch_main(a, p, y_f32 != 0, false, st);
   if (p.splits > 1) {
     const long long n4 = (long long)M * (N / 4);
     const unsigned blocks = (unsigned)((n4 + 255) / 256);
@@ -968,19 +1397,10 @@ extern "C" int fqa_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, 
   return hipGetLastError() == hipSuccess ? FQA_OK : FQA_ELAUNCH;
 }
 
-// The argmax plan: the projection's tiles without a K split (every tile sees whole rows
-// of its columns).
-static bool argmax_plan(int32_t M, int32_t N, int32_t K, GemmPlan& p) {
-  if (!gemm_shape_ok(M, N, K) || M == 0) return false;
-  p = gemm_plan(M, N, K);
-  p.splits = 1;
-  return true;
-}
-
 extern "C" int64_t fqa_gemm_argmax_workspace_bytes(int32_t M, int32_t N, int32_t K) {
-  GemmPlan p;
-  if (!argmax_plan(M, N, K, p)) return 0;
-  return (int64_t)p.n_tiles * M * 8;
+  // a pair per row and column tile, sized for tiles of 128 columns, above 1024 rows of 256
+  if (!gemm_shape_ok(M, N, K) || M == 0) return 0;
+  return (int64_t)(N / (M > 1024 && N % 256 == 0 ? 256 : 128)) * M * 8;
 }
 
 extern "C" int fqa_gemm_argmax(const void* x, int64_t ldx, const void* w, int64_t ldw,
@@ -994,9 +1414,11 @@ extern "C" int fqa_gemm_argmax(const void* x, int64_t ldx, const void* w, int64_
   if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)workspace & 15)) return FQA_EINVAL;
   if ((int64_t)(M - 1) * ldx * 2 >= (int64_t)1 << 32 || (int64_t)(N - 1) * ldw * 2 >= (int64_t)1 << 32)
     return FQA_EUNSUPPORTED;
-  GemmPlan p;
-  argmax_plan(M, N, K, p);
-  if (workspace_bytes < (int64_t)p.n_tiles * M * 8) return FQA_EINVAL;
+  // without a K split (every tile sees whole rows of its columns)
+  GemmPlan p = gemm_plan(M, N, K, 1);
+  if (M > 1024 && N % 256 == 0 && p.bn != 256)  // as the workspace is sized
+    p = GemmPlan{kTileL, 256, 256, 1, (M + 255) / 256, N / 256};
+  if (workspace_bytes < fqa_gemm_argmax_workspace_bytes(M, N, K)) return FQA_EINVAL;
   if ((int64_t)p.m_tiles * p.n_tiles > 0x7fffffff) return FQA_EINVAL;
   GemmArgs a{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), nullptr, nullptr,
              ldx, ldw, 0, M, N, K, 1, p.m_tiles, p.n_tiles,
@@ -1004,10 +1426,10 @@ extern "C" int fqa_gemm_argmax(const void* x, int64_t ldx, const void* w, int64_
              reinterpret_cast<int*>(static_cast<char*>(workspace) + (int64_t)p.n_tiles * M * 4)};
   hipStream_t st = (hipStream_t)stream;
   switch (p.tile) {
-    case 0: launch_argmax<TileL>(a, st); break;
-    case 4: launch_argmax<TileL8>(a, st); break;
-    case 1: launch_argmax<TileM>(a, st); break;
-    case 2: launch_argmax<TileS>(a, st); break;
+    case kTileL: launch_argmax<TileL>(a, st); break;
+    case kTileH: launch_argmax<TileH>(a, st); break;
+    case kTileM: launch_argmax<TileM>(a, st); break;
+    case kTileS: launch_argmax<TileS>(a, st); break;
     default: launch_argmax<TileT>(a, st); break;
   }
   hipLaunchKernelGGL(gemm_argmax_reduce_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, st, a,

@@ -23,16 +23,16 @@ struct GemmAppend {
   int write_k;
 };
 
-// y = x . W^T with fqa_gemm's argument rules.  When the plan splits K, only the split
-// kernel runs: the fp32 partials land in `workspace` as [splits][M][N] and the caller
-// consumes them (in split order, as fqa_gemm's reduction does); otherwise bf16 y is
-// written.  Returns the number of splits (>= 1), 0 for M = 0, or an FQA_E code.
-// With `app` (N = 6144, y = the qkv buffer), an unsplit plan on the 256-row tiles applies
-// the per-head norm + RoPE + paged append in its epilogue instead of writing bf16 y, with
-// the results fqa_qknorm_rope_append would give on that y; *appended says so.
+// The QKV projection x . W^T (N = 6144, y = the qkv buffer) with fqa_gemm's argument rules
+// and plan, for a caller that appends.  An unsplit plan on the 128- and 256-row tiles applies
+// `app` (the per-head norm + RoPE + paged append) in its epilogue, with the results
+// fqa_qknorm_rope_append would give on fqa_gemm's y; *appended says so.  Otherwise the fp32
+// partials land in `workspace` as [planes][M][N], to be summed in plane order as fqa_gemm's
+// reduction does, and y is not written.  Returns the number of planes, 0 for M = 0 or when
+// appended, or an FQA_E code.
 int gemm_launch_partials(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
                          int64_t ldy, int32_t M, int32_t N, int32_t K, void* workspace,
                          int64_t workspace_bytes, hipStream_t st,
-                         const GemmAppend* app = nullptr, bool* appended = nullptr);
+                         const GemmAppend& app, bool* appended);
 
 }  // namespace fqa

@@ -22,7 +22,7 @@
 // page's rows (except where a range ends) go through the same XCD's L2.
 // Memory-bound: per row 12 KiB read, 8 KiB (q) + 4 KiB (k, v) written.
 //
-// fqa_qkv_proj_append runs the same kernel on the QKV projection's split-K partials
+// fqa_qkv_proj_append runs the same kernel on the QKV projection's fp32 partials
 // (kPart): a row's values are the sum of the fp32 partials in split order, rounded to
 // bf16 exactly as the projection's own reduction would round them, so the results match
 // fqa_gemm + fqa_qknorm_rope_append bit for bit without the bf16 qkv round trip.
@@ -341,13 +341,12 @@ extern "C" int fqa_qkv_proj_append(const fqa_dims* dims, const uint16_t* x, int6
   const GemmAppend app{q_norm_w, k_norm_w, cos_tab, sin_tab, rope_max_pos, positions,
                        slot_mapping, meta, pool, pool_pages, dims->eps, write_k_inplace};
   bool appended = false;
-  const int splits = gemm_launch_partials(x, ldx, w_qkv, ldw, qkv, dims->qkv_stride, rows,
-                                          kQkvStride, hidden, workspace, workspace_bytes, st,
-                                          &app, &appended);
-  if (splits < 0) return splits;
+  const int planes = gemm_launch_partials(x, ldx, w_qkv, ldw, qkv, dims->qkv_stride, rows,
+                                          kQkvStride, hidden, workspace, workspace_bytes, st, app,
+                                          &appended);
+  if (planes < 0) return planes;
   if (appended) return hipGetLastError() == hipSuccess ? FQA_OK : FQA_ELAUNCH;
   return append_launch(dims, qkv, q_norm_w, k_norm_w, cos_tab, sin_tab, rope_max_pos, positions,
                        slot_mapping, meta, rows, pool, pool_pages, write_k_inplace,
-                       splits > 1 ? static_cast<const float*>(workspace) : nullptr, splits, rows,
-                       st);
+                       static_cast<const float*>(workspace), planes, rows, st);
 }

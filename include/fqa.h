@@ -449,8 +449,8 @@ int fqa_sample(const float* logits, int32_t n_rows, int32_t vocab, int64_t row_s
  * lm_head); fp32 accumulation.  Requires N % 128 == 0 and K % 64 == 0 (FQA_EUNSUPPORTED
  * otherwise: every Qwen3-8B projection qualifies), ldx and ldw multiples of 8 and ldy of 4
  * elements, x, W and y 16-byte aligned, and every row start of x and W within 4 GiB of
- * its base.  Shapes with few 256 x 128 output tiles split K over several workgroups and
- * need `workspace` (16-byte aligned) of fqa_gemm_workspace_bytes(M, N, K) bytes (0: none;
+ * its base.  Shapes with few output tiles may split K over several workgroups and need
+ * `workspace` (16-byte aligned) of fqa_gemm_workspace_bytes(M, N, K) bytes (0: none;
  * its contents need no initialisation).  M = 0 is a no-op. */
 int64_t fqa_gemm_workspace_bytes(int32_t M, int32_t N, int32_t K);
 int fqa_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy,
@@ -461,10 +461,10 @@ int fqa_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, in
  * model_runtime.cu:322-325, kernels.cu:184-327): out[m] = the column of the largest value of
  * row m of x . W^T (fp32 accumulation over the whole of K per tile, never split), ties and
  * rows without a value above -1e30 resolved as fqa_sample's greedy rows resolve them.  Where
- * fqa_gemm's plan for the same shape does not split K (every lm_head shape: 1187 column
+ * fqa_gemm_workspace_bytes is 0 for the same shape (every lm_head shape: 1187 column
  * tiles at vocab 151936), the values are the fp32 logits fqa_gemm writes with y_f32 = 1,
- * so the pick equals fqa_sample's greedy pick on those logits; where fqa_gemm splits K its
- * logits are summed in another order and can differ in the last bit.  Every row of x is
+ * so the pick equals fqa_sample's greedy pick on those logits; elsewhere fqa_gemm may sum its
+ * logits in another order, and they can differ in the last bit.  Every row of x is
  * picked greedily: in a batch that mixes greedy and sampled rows, either gather the greedy
  * rows of x into a compact x first, or pick every row and then run fqa_gemm (fp32) +
  * fqa_sample on the sampled rows only and let their picks overwrite.
@@ -482,11 +482,10 @@ int fqa_gemm_argmax(const void* x, int64_t ldx, const void* w, int64_t ldw, int3
  * per row the norm + RoPE + append of fqa_qknorm_rope_append with the same arguments and
  * results (rows_bound = rows; meta[FQA_META_ROWS] must not exceed rows).  The bf16 qkv of
  * the unfused path is never written and read back:
- *   - when the projection splits K (decode-sized row counts), the append kernel reads the
- *     fp32 split partials directly, summed in the order fqa_gemm's reduction uses;
- *   - otherwise (513..1024 rows, and from 1281 rows on: the tiles alone fill the device)
- *     the projection's epilogue rounds its tile to bf16 in LDS and applies the norm, RoPE
- *     and append there.
+ *   - where the projection leaves fp32 sums (decode-sized row counts, or K split), the
+ *     append kernel reads them directly, in the order fqa_gemm's reduction uses;
+ *   - otherwise (from ~257 rows on: the tiles alone fill the device) the projection's
+ *     epilogue rounds its tile to bf16 in LDS and applies the norm, RoPE and append there.
  * Either way the results are bit-identical to fqa_gemm followed by fqa_qknorm_rope_append,
  * and only q (and k with write_k_inplace) of qkv is written, for rows below
  * meta[FQA_META_ROWS]; v goes to the pool only.  workspace: fqa_gemm_workspace_bytes(rows,

@@ -89,7 +89,7 @@ def test_gemm_smaller_workspace(gpu):
 @pytest.mark.parametrize("M,K,write_k,rows", [
     (100, 64, 1, None),     # one k step: the 128-row tile's append epilogue
     (129, 1024, 0, None),   # a slab's fp32 sums through the append kernel
-    (300, 1024, 0, None),   # 128 x 128 tiles
+    (345, 1024, 0, None),   # 128 x 128 tiles
     (450, 1024, 1, 440),    # ... with the row count inside the last one
     (700, 512, 1, 690),     # 256 x 128 tiles
 ])

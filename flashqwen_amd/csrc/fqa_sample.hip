@@ -7,20 +7,31 @@
 // first index at which the running kept mass reaches u * (kept mass).
 //
 // MI355X design: one 1024-thread workgroup per row.  Wave w owns a contiguous segment of
-// the row and its lanes read consecutive elements (coalesced 256-byte wave loads), so
-// index order is (segment, step, lane) and the inverse-CDF pick keeps vocabulary order.
-// The reference finds the top-p threshold by 32 bisection passes over the row, each
-// recomputing every weight; here it is a 3-level radix select on the weights' float bits
-// (bits 30..20, 19..9, 8..0; positive floats order like their bit patterns), with exact
-// integer mass histograms in LDS: the exact smallest kept weight after 3 levels, and with
-// it each wave's kept mass.  A top-p row is read 3 times in full (max + sum, level 1, level 2): level 2 also
-// copies the weights of the boundary bin into LDS, and level 3 runs on that copy.  Only
-// when the boundary bin holds more than 16384 weights is the row read a 4th time for level
-// 3.  A temperature-only row is read once (its kept mass per wave is the rescaled pass-1
-// sum), against 35 reads in the reference; the pick then reads 1/16 of one wave's segment
-// twice.
-
+// the row and its lanes read 16 bytes each (1 KiB wave loads), so index order is (segment,
+// step, lane, element) and the inverse-CDF pick keeps vocabulary order.  The reference finds
+// the top-p threshold by 32 bisection passes over the row, each recomputing every weight;
+// here it is a 3-level radix select on the weights' float bits (bits 30..20, 19..9, 8..0;
+// positive floats order like their bit patterns), with exact integer mass histograms in LDS:
+// the exact smallest kept weight after 3 levels, and with it each wave's kept mass.  A top-p
+// row is read 3 times in full (max + sum, level 1, and a pass that copies the weights of the
+// boundary bin into LDS, on which levels 2 and 3 run).  Only when the boundary bin may hold
+// more than 16384 weights is the row read a 4th time for level 3, and once more where the
+// boundary lies below 2^-31 of the largest weight.  A temperature-only row is read once (its
+// kept mass per wave is the rescaled pass-1 sum); the pick then reads 1/16 of one wave's
+// segment.
+//
+// What bounds it: with a workgroup per row, what one CU loads and computes.  Each wave keeps
+// 4 KiB of loads in flight while it works on the 4 KiB before (128 KiB per CU; 2 KiB with no
+// overlap made a pass ~20 us however few the rows), and per-element work is kept free of
+// branches and of atomics that meet: the running maximum is selected, not branched on, level
+// 1 has a column per lane, room in the copy is taken once per 4 KiB.  Sums keep one order
+// (lane, step, element; then lanes; then waves), so a draw near a cumulative-mass boundary
+// falls the same way.  151936 logits, 4 rows: greedy 21.6 -> 13.7 us, temperature 27.6 -> 20.1,
+// top-p 0.9 71 -> 61, nearly flat rows 185 -> 76; 256 rows: 32.7 -> 32.0, 37.4 -> 36.6, 93 ->
+// 93 (HBM and the caches carry the reads there), 207 -> 115.
 #include "fqa_common.h"
+
+#include <cfloat>
 
 namespace fqa {
 namespace {
@@ -28,7 +39,10 @@ namespace {
 constexpr int kSThreads = 1024;
 constexpr int kSWaves = kSThreads / kWave;
 constexpr int kBins = 2048;  // histogram bins per radix level (levels use 11, 11, 9 bits)
-constexpr int kChunk = 2;    // 256-element steps whose loads a wave issues back to back
+constexpr int kChunk = 4;    // 256-element steps whose loads a wave issues back to back
+constexpr int kCols = 256;   // level-1 bins with a column per lane: the 31 octaves below 1
+constexpr int kCol0 = (127 << 3) + 8 - kCols;  // ... from this bin on (bits 30..20)
+constexpr int kCandCap = 16384;  // boundary-bin weights that the LDS copy holds
 // Histogram masses are exact integers: a weight with exponent field E adds its 24-bit
 // significand, and a bin's mass is that sum times 2^(max(E, 1) - 150) (every bin holds one
 // exponent).  ds_add_u64 runs at several times the rate of ds_add_f32 on gfx950, whose
@@ -54,6 +68,11 @@ struct SampArgs {
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
   return v;
 }
 // Inclusive prefix sum over the wave's lanes.
@@ -103,24 +122,19 @@ __device__ int find_crossing(const float* hist, int nbins, float above, float ne
   return *sres;
 }
 
-// Wave w of the row covers [seg0, seg1), a whole number of 256-element steps except at
-// the row's end; in a step lane l holds elements s0 + 4l .. s0 + 4l + 3, so vocabulary
-// order is (wave, step, lane, element).  With kVec4 (16-byte aligned rows) a lane loads its
-// 4 logits as one float4: a wave load moves 1 KiB.
-template <bool kVec4>
+// Elements i .. i + 3 of the row (those past `end` as -inf: weight 0, never the largest).
 __device__ __forceinline__ void load4(const float* lg, int i, int end, float (&x)[4]) {
-  if (kVec4 && i + 3 < end) {
-    const float4 v = *reinterpret_cast<const float4*>(lg + i);
-    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+  if (i + 3 < end) {
+    __builtin_memcpy(x, lg + i, 16);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = i + e < end ? lg[i + e] : -INFINITY;
   }
 }
 
-template <bool kVec4>
+typedef float Chunk[kChunk][4];
+
 __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
-  __shared__ float hist[kBins];
   __shared__ float sh[kSWaves];
   __shared__ float sh2[kSWaves];
   __shared__ int sres;
@@ -130,49 +144,66 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
   const int row = blockIdx.x;
   const int N = a.vocab;
   const float* lg = a.logits + (long long)row * a.stride;
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t >> 6;
-  constexpr int kStep = 4 * kWave;
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  // Wave w of the row covers [seg0, seg1), a whole number of 256-element steps except at
+  // the row's end; in a step lane l holds elements s0 + 4l .. s0 + 4l + 3.
+  constexpr int kStep = 4 * kWave, kSpan = kChunk * kStep;
   const int seg = ((N + kSWaves * kStep - 1) / (kSWaves * kStep)) * kStep;
   const int seg0 = min(w * seg, N), seg1 = min(seg0 + seg, N);
   const float it = a.inv_temp[row];
-  // calls f(index, logit) for this lane's elements, in vocabulary order per lane.  The
-  // segment is walked in chunks of kChunk steps whose loads are all issued before any
-  // element is used, so a wave keeps kChunk KiB in flight instead of waiting out one
-  // load's latency per step.
-  auto for_each = [&](auto&& f) {
-    for (int c0 = seg0; c0 < seg1; c0 += kChunk * kStep) {
-      float x[kChunk][4];
-      if (kVec4 && c0 + kChunk * kStep <= seg1) {
+  // f(chunk, its first index) for the segment's chunks of kChunk steps, in order; a chunk's
+  // loads are issued before the chunk before it is used.
+  auto load_chunk = [&](Chunk& x, int c0, int end) {
+    if (c0 + kSpan <= end) {
 #pragma unroll
-        for (int u = 0; u < kChunk; ++u) {
-          const float4 v = *reinterpret_cast<const float4*>(lg + c0 + u * kStep + 4 * lane);
-          x[u][0] = v.x; x[u][1] = v.y; x[u][2] = v.z; x[u][3] = v.w;
-        }
-      } else {
+      for (int u = 0; u < kChunk; ++u) __builtin_memcpy(x[u], lg + c0 + u * kStep + 4 * lane, 16);
+    } else {
 #pragma unroll
-        for (int u = 0; u < kChunk; ++u) load4<kVec4>(lg, c0 + u * kStep + 4 * lane, seg1, x[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kChunk; ++u) {
-        const int i = c0 + u * kStep + 4 * lane;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (i + e < seg1) f(i + e, x[u][e]);
-      }
+      for (int u = 0; u < kChunk; ++u) load4(lg, c0 + u * kStep + 4 * lane, end, x[u]);
     }
+  };
+  auto for_chunks = [&](auto&& f) {
+    if (seg0 >= seg1) return;
+    Chunk x, next;
+    load_chunk(x, seg0, seg1);
+    for (int c0 = seg0; c0 < seg1; c0 += kSpan) {
+      if (c0 + kSpan < seg1) load_chunk(next, c0 + kSpan, seg1);
+      f(x, c0);
+#pragma unroll
+      for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[u][e] = next[u][e];
+    }
+  };
+  auto chunk_max = [](const Chunk& x) {
+    float m = x[0][0];
+#pragma unroll
+    for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = fmaxf(m, x[u][e]);
+    return m;
   };
 
   if (it <= 0.f) {  // greedy: largest logit, the reference's tie order (greedy_key)
-    float best = -INFINITY;
+    float best = -INFINITY, wave_best = -INFINITY;  // this lane's, the wave's
     int bi = N;
     uint32_t bk = 0xffffffffu;
-    for_each([&](int i, float v) {
-      const uint32_t k = greedy_key(i);
-      if (v > best || (v == best && k < bk)) {
-        best = v;
-        bi = i;
-        bk = k;
-      }
+    for_chunks([&](const Chunk& x, int c0) {
+      if (!__any(chunk_max(x) >= wave_best)) return;  // soon the usual case
+#pragma unroll
+      for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = c0 + u * kStep + 4 * lane + e;
+          const uint32_t k = greedy_key(i);
+          if (x[u][e] > best || (x[u][e] == best && k < bk)) {
+            best = x[u][e];
+            bi = i;
+            bk = k;
+          }
+        }
+      wave_best = wave_max(best);
     });
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -209,22 +240,24 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
   }
 
   // pass 1: row max and total weight together (online: the running sum is rescaled when
-  // the running max grows), merged across lanes and waves the same way
-  float lm = -INFINITY, ls = 0.f;
-  for_each([&](int, float v) {
-    if (v == -INFINITY) return;  // a masked token weighs 0 (and -inf - -inf is NaN)
-    if (v > lm) {
-      ls = ls * __expf((lm - v) * it) + 1.f;
-      lm = v;
-    } else {
-      ls += __expf((v - lm) * it);
-    }
+  // the running max grows), merged across lanes and waves the same way.  The running max
+  // starts at the lowest finite value, so a masked token (-inf) weighs 0 (exp2(-inf)).
+  float lm = -FLT_MAX, ls = 0.f;
+  for_chunks([&](const Chunk& x, int) {
+#pragma unroll
+    for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = x[u][e];
+        const float w1 = __expf(-fabsf(v - lm) * it);  // of the smaller of the two
+        ls = v > lm ? fmaf(ls, w1, 1.f) : ls + w1;
+        lm = fmaxf(lm, v);
+      }
   });
   auto merge = [&](float& m0, float& s0v, float m1, float s1) {
+#pragma clang fp contract(off)
     const float mn = fmaxf(m0, m1);
-    if (mn == -INFINITY) return;
-    s0v = (m0 == -INFINITY ? 0.f : s0v * __expf((m0 - mn) * it)) +
-          (m1 == -INFINITY ? 0.f : s1 * __expf((m1 - mn) * it));
+    s0v = s0v * __expf((m0 - mn) * it) + s1 * __expf((m1 - mn) * it);
     m0 = mn;
   };
 #pragma unroll
@@ -240,10 +273,14 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
 
   // skm[w]: the kept mass of wave w's segment
   __shared__ float skm[kSWaves];
-  __shared__ unsigned long long hcnt[kBins];         // levels 1 and 2
-  __shared__ unsigned long long hcnt3[kSWaves][512];  // level 3, one per wave
+  // level 1 with a column per lane, then the copied boundary weights and a spare word per
+  // lane, or level 3 per wave
+  __shared__ unsigned long long big[kCols * kWave];
+  __shared__ unsigned long long hcnt[kBins];
+  __shared__ float hist[kBins];
   __shared__ unsigned long long s_kmc[kSWaves];
   __shared__ int s_ncand;
+  static_assert((kCandCap + kWave) * 4 <= kCols * kWave * 8 && kSWaves * 512 <= kCols * kWave, "big");
   uint32_t thr = 0;  // kept: weights whose bits are >= thr (all, without top-p)
   const float tp = a.top_p[row];
   if (tp < 1.f) {
@@ -252,47 +289,122 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
     // (1 - top_p) * Z / 2, so the top-p boundary lies above them.
     const float need = fmaxf(tp * Z, 1e-37f);  // top_p = 0 still keeps the largest weight
     const float x_min = 0.5f * (1.f - tp) * Z / (float)N;
-    for (int b = t; b < kBins; b += kSThreads) hcnt[b] = 0ull;
+    for (int b = t; b < kCols * kWave; b += kSThreads) big[b] = 0ull;
+    for (int b = t; b < kBins; b += kSThreads) {
+      hcnt[b] = 0ull;
+      hist[b] = 0.f;
+    }
     __syncthreads();
-    for_each([&](int, float v) {
-      const uint32_t bits = __float_as_uint(weight(v));
-      if (__uint_as_float(bits) >= x_min) atomicAdd(&hcnt[(bits >> 20) & 2047], significand(bits));
+    for_chunks([&](const Chunk& x, int) {
+#pragma unroll
+      for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t bits = __float_as_uint(weight(x[u][e]));
+          const int b = (int)(bits >> 20) - kCol0;
+          if (b >= 0 && __uint_as_float(bits) >= x_min)
+            atomicAdd(&big[b * kWave + lane], significand(bits));
+        }
     });
     __syncthreads();
-    for (int b = t; b < kBins; b += kSThreads) hist[b] = bin_mass(hcnt[b], b >> 3);
+    {  // bin b's columns, 16 per thread
+      const unsigned long long* src = big + t * 16;
+      unsigned long long c = 0;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) c += src[(k + t) & 15];
+      c += __shfl_xor(c, 1, kWave);
+      c += __shfl_xor(c, 2, kWave);
+      if ((t & 3) == 0) {
+        const int b = kCol0 + (t >> 2);
+        hcnt[b] = c;
+        hist[b] = bin_mass(c, b >> 3);
+      }
+    }
     __syncthreads();
     float above;
-    const int b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
+    int b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
+    if (b1 < kCol0) {
+      // the boundary lies further down (top_p within 2^-31 or so of 1, or rounding): the
+      // bins below the columns too
+      for_chunks([&](const Chunk& x, int) {
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t bits = __float_as_uint(weight(x[u][e]));
+            const int b = (int)(bits >> 20);
+            if (b < kCol0 && __uint_as_float(bits) >= x_min) atomicAdd(&hcnt[b], significand(bits));
+          }
+      });
+      __syncthreads();
+      for (int b = t; b < kBins; b += kSThreads) hist[b] = bin_mass(hcnt[b], b >> 3);
+      __syncthreads();
+      b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
+    }
     const int e1 = b1 >> 3;  // the exponent field of every weight in bin b1
-    // pass 3: level 2, bits 19..9 of the weights in bin b1.  The same pass sums, per
-    // lane, the weights above bin b1 (all kept) and copies the weights in bin b1 into LDS
-    // (low 20 bits and the wave, in the level-3 histograms' memory); when they all fit,
-    // level 3 and the kept masses come from that copy and the row is not read again.
-    uint32_t* cand = reinterpret_cast<uint32_t*>(&hcnt3[0][0]);
-    constexpr int kCandCap = kSWaves * 512 * 2;
+    // A normal weight's significand is 2^23 or more, so this bin's weights fit the copy.
+    const bool copy = e1 > 0 && (hcnt[b1] >> 23) <= kCandCap;
+    // pass 3: per lane, the mass of the weights above bin b1 (all kept), and the weights in
+    // bin b1 copied into LDS (low 20 bits and the wave), on which level 2 (bits 19..9),
+    // level 3 and the kept masses run without reading the row again; or level 2 here.
+    uint32_t* cand = reinterpret_cast<uint32_t*>(big);
+    __syncthreads();
     for (int b = t; b < kBins; b += kSThreads) hcnt[b] = 0ull;
     if (t == 0) s_ncand = 0;
     __syncthreads();
     float km1 = 0.f;
-    for_each([&](int, float v) {
-      const float wv = weight(v);
-      const uint32_t bits = __float_as_uint(wv);
-      const int bb = (int)(bits >> 20);
-      if (bb > b1) {
-        km1 += wv;
-      } else if (bb == b1) {
-        atomicAdd(&hcnt[(bits >> 9) & 2047], significand(bits));
-        const int slot = atomicAdd(&s_ncand, 1);
-        if (slot < kCandCap) cand[slot] = ((uint32_t)w << 20) | (bits & 0xfffffu);
+    for_chunks([&](const Chunk& x, int) {
+      uint32_t bits[kChunk][4];
+      int n = 0;
+#pragma unroll
+      for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float wv = weight(x[u][e]);
+          bits[u][e] = __float_as_uint(wv);
+          const int bb = (int)(bits[u][e] >> 20);
+          km1 += bb > b1 ? wv : 0.f;
+          n += bb == b1 ? 1 : 0;
+        }
+      if (!__any(n > 0)) return;
+      if (copy) {
+        // room for this lane's n weights: one addition per wave; then without branches,
+        // what is not copied goes to a spare word
+        const int incl = wave_incl_scan(n);
+        int base = 0;
+        if (lane == kWave - 1) base = atomicAdd(&s_ncand, incl);
+        int slot = __builtin_amdgcn_readlane(base, kWave - 1) + incl - n;
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const bool in = (int)(bits[u][e] >> 20) == b1;
+            cand[in ? slot : kCandCap + lane] = ((uint32_t)w << 20) | (bits[u][e] & 0xfffffu);
+            slot += in ? 1 : 0;
+          }
+      } else {
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if ((int)(bits[u][e] >> 20) == b1)
+              atomicAdd(&hcnt[(bits[u][e] >> 9) & 2047], significand(bits[u][e]));
       }
     });
     __syncthreads();
+    const int nc = copy ? s_ncand : 0;
+    if (copy) {
+      for (int i = t; i < nc; i += kSThreads) {
+        const uint32_t bits = ((uint32_t)b1 << 20) | (cand[i] & 0xfffffu);
+        atomicAdd(&hcnt[(bits >> 9) & 2047], significand(bits));
+      }
+      __syncthreads();
+    }
     for (int b = t; b < kBins; b += kSThreads) hist[b] = bin_mass(hcnt[b], e1);
     __syncthreads();
     const int b2 = find_crossing(hist, kBins, above, need, sh, &sres, &sres_f, &above);
     const uint32_t hi = ((uint32_t)b1 << 11) | (uint32_t)b2;
-    const int nc = s_ncand;
-    if (nc <= kCandCap) {
+    if (copy) {
       // level 3 over the copied weights of (b1, b2), then each wave's kept mass: the
       // weights above bin b1 plus its copied weights at or above the threshold
       for (int b = t; b < 512; b += kSThreads) hcnt[b] = 0ull;
@@ -318,34 +430,38 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
       // pass 4: level 3 (bits 8..0 of the weights in (b1, b2)) as one histogram per
       // wave, and per wave the mass of the weights above (b1, b2), which are all kept:
       // the kept mass per wave then follows from the histograms without another pass
-      unsigned long long* h3 = &hcnt3[0][0];
-      for (int b = t; b < kSWaves * 512; b += kSThreads) h3[b] = 0ull;
+      for (int b = t; b < kSWaves * 512; b += kSThreads) big[b] = 0ull;
       __syncthreads();
       float km_hi = 0.f;
-      for_each([&](int, float v) {
-        const float wv = weight(v);
-        const uint32_t bits = __float_as_uint(wv);
-        if ((bits >> 9) > hi) km_hi += wv;
-        else if ((bits >> 9) == hi) atomicAdd(&hcnt3[w][bits & 511], significand(bits));
+      for_chunks([&](const Chunk& x, int) {
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float wv = weight(x[u][e]);
+            const uint32_t bits = __float_as_uint(wv);
+            if ((bits >> 9) > hi) km_hi += wv;
+            else if ((bits >> 9) == hi) atomicAdd(&big[w * 512 + (bits & 511)], significand(bits));
+          }
       });
       __syncthreads();
       if (t < 512) {
         unsigned long long c = 0;
-        for (int k = 0; k < kSWaves; ++k) c += hcnt3[k][t];
+        for (int k = 0; k < kSWaves; ++k) c += big[k * 512 + t];
         hist[t] = bin_mass(c, e1);
       }
       __syncthreads();
       const int b3 = find_crossing(hist, 512, above, need, sh, &sres, &sres_f, &above);
       thr = (hi << 9) | (uint32_t)b3;
       unsigned long long c = 0;
-      for (int b = b3 + lane; b < 512; b += kWave) c += hcnt3[w][b];
+      for (int b = b3 + lane; b < 512; b += kWave) c += big[w * 512 + b];
       float km = km_hi + bin_mass(c, e1);
       km = wave_sum(km);
       if (lane == 0) skm[w] = km;
     }
   } else {
     // every weight is kept: wave w's mass is its pass-1 sum rescaled to the row max
-    if (t < kSWaves) skm[t] = sh[t] == -INFINITY ? 0.f : sh2[t] * __expf((sh[t] - m) * it);
+    if (t < kSWaves) skm[t] = sh2[t] * __expf((sh[t] - m) * it);
   }
   __syncthreads();
 
@@ -379,14 +495,21 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
   const int S0 = min(ws * seg, N), S1 = min(S0 + seg, N);
   const int sub = ((S1 - S0 + kSWaves * kStep - 1) / (kSWaves * kStep)) * kStep;
   const int u0 = min(S0 + w * sub, S1), u1 = min(u0 + sub, S1);
+  // this wave's sub-segment; its first chunk stays in registers for the walk
+  Chunk first_x;
+  load_chunk(first_x, u0, u1);
   float m2 = 0.f;
-  for (int s0 = u0; s0 < u1; s0 += kStep) {
-    const int i = s0 + 4 * lane;
-    float x[4];
-    load4<kVec4>(lg, i, u1, x);
+  auto add_kept = [&](const Chunk& x) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i + e < u1) m2 += kept(x[e]);
+    for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m2 += kept(x[u][e]);
+  };
+  add_kept(first_x);
+  for (int c0 = u0 + kSpan; c0 < u1; c0 += kSpan) {
+    Chunk x;
+    load_chunk(x, c0, u1);
+    add_kept(x);
   }
   m2 = wave_sum(m2);
   if (lane == 0) sh2[w] = m2;
@@ -416,7 +539,17 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
     for (int s0 = u0; s0 < u1; s0 += kStep) {
       const int i = s0 + 4 * lane;
       float x[4], kw[4];
-      load4<kVec4>(lg, i, u1, x);
+      if (s0 - u0 < kSpan) {
+        const int q = (s0 - u0) / kStep;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = first_x[0][e];
+#pragma unroll
+        for (int u = 1; u < kChunk; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = q == u ? first_x[u][e] : x[e];
+      } else {
+        load4(lg, i, u1, x);
+      }
       float lsum = 0.f;
       int llast = -1;
 #pragma unroll
@@ -468,12 +601,7 @@ extern "C" int fqa_sample(const float* logits, int32_t n_rows, int32_t vocab,
   if (n_rows == 0) return FQA_OK;
   if (!logits || !inv_temp || !top_p || !u || !out) return FQA_EINVAL;
   SampArgs a{logits, vocab, row_stride, inv_temp, top_p, u, out};
-  const bool vec4 = ((uintptr_t)logits & 15) == 0 && (row_stride & 3) == 0;
-  if (vec4)
-    hipLaunchKernelGGL(sample_kernel<true>, dim3((unsigned)n_rows), dim3(kSThreads), 0,
-                       (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(sample_kernel<false>, dim3((unsigned)n_rows), dim3(kSThreads), 0,
-                       (hipStream_t)stream, a);
+  hipLaunchKernelGGL(sample_kernel, dim3((unsigned)n_rows), dim3(kSThreads), 0,
+                     (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? FQA_OK : FQA_ELAUNCH;
 }

@@ -7,7 +7,7 @@
 //
 // MI355X design:
 //  * Four kernels, chosen by a model of their times (gemm_plan):
-//    - gemm_quad_kernel: tiles of 256 x 256, 256 x 128 and 128 x 128 on 4 waves, one per SIMD;
+//    - gemm_quad_kernel: tiles of 128 to 256 rows and columns on 4 waves, one per SIMD;
 //    - gemm_slab_kernel: up to 96 x 64 outputs per workgroup for few rows, its waves dividing K
 //      and summing in LDS, so that decode steps fill the CUs without a second kernel;
 //    - gemm_kernel: 32 and 64 rows by 128 columns where W is wide enough to fill the CUs;
@@ -95,6 +95,8 @@ constexpr bool kIsQuad = false;
 template <int M, int N, int R>
 constexpr bool kIsQuad<Quad<M, N, R>> = true;
 using TileL = Quad<256, 256, 2>;
+using TileP = Quad<192, 256, 2>;
+using TileQ = Quad<256, 192, 2>;
 using TileH = Quad<256, 128, 3>;
 using TileM = Quad<128, 128, 5>;
 using TileS = Tile<1, 4, 2, 1, 6>;  // 64 x 128
@@ -347,6 +349,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& a, char* lds,
     constexpr int kRowChunks = T::kBN / 8, kRows = kWave / kRowChunks;  // rows per store
     for (int r0 = kRows * w; r0 < T::kBM; r0 += kRows * T::kWaves) {
       const int r = r0 + lane / kRowChunks, c = lane % kRowChunks, m = row0 + r;
+      if (lane >= kRows * kRowChunks) break;  // 192 columns: 2 rows on 48 lanes
       const uint4 v = *reinterpret_cast<const uint4*>(lds + r * kTilePitch<T> + c * 16);
       if (m >= a.M) continue;
       uint16_t* d = y + m * a.ldy + c * 8;
@@ -1170,7 +1173,7 @@ bool slab_dispatch(int i, F&& f) {
 }
 
 // The launch plan of one call.
-enum Tiles { kTileT, kTileS, kTileM, kTileH, kTileL, kSlab0 };
+enum Tiles { kTileT, kTileS, kTileM, kTileH, kTileQ, kTileP, kTileL, kSlab0 };
 struct GemmPlan {
   int tile;  // Tiles; kSlab0 + i: kSlabs[i]
   int bm, bn, splits, m_tiles, n_tiles;
@@ -1180,8 +1183,12 @@ struct GemmPlan {
 // 24576 x 4096 and 4096 x 12288 at 6 to 2048 rows with W cold (within ~15% of each, and
 // nearly always the measured order):
 //  * Tiles of 128 columns or more: 2.4 for the launch and, per round of 256 workgroups, 5 to
-//    start and store and 1.29 (256 x 256), 0.78 (256 x 128) or 0.45 (128 x 128; 0.75 with a
-//    single row tile, whose W comes from HBM) per step of 64 k.
+//    start and store and, per step of 64 k, 1.29 (256 x 256), 1.03 (192 x 256, 256 x 192; 1.24
+//    with K split), 0.78 (256 x 128) or 0.45 (128 x 128; 0.58 with K split, 0.75 with a single
+//    row tile, whose W comes from HBM).  What decides between them is mostly how full the
+//    last round is: gate_up at 384 / 700 / 1000 / 1500 rows 90 / 154 / 178 / 260 us without
+//    the 192-wide tiles, 80 / 141 / 164 / 238 with them; qkv at 1500 rows 77 -> 68, down 139 ->
+//    127.
 //  * Slabs: 6, 1 per 70 KB that a workgroup stages and 1 per 4096 outputs of the tile (the
 //    sum over its waves); one round of workgroups; for x that fits an XCD's L2
 //    beside the W stream (3.5 MB: at 12288 k and 160 rows the slabs lose).
@@ -1206,14 +1213,22 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
       best = p;
     }
   };
-  const int quads[3][3] = {{kTileL, 256, 256}, {kTileH, 256, 128}, {kTileM, 128, 128}};
+  // (256 x 192 tiles cut heads: not at the QKV width, whose epilogue may append)
+  const struct {
+    int tile, bm, bn;
+    float step, split_step;
+  } quads[] = {{kTileL, 256, 256, 1.29f, 1.29f},
+               {kTileP, 192, 256, 1.03f, 1.24f},
+               {kTileQ, 256, 192, 1.03f, 1.24f},
+               {kTileH, 256, 128, 0.78f, 0.78f},
+               {kTileM, 128, 128, 0.45f, 0.58f}};
   for (const auto& q : quads) {
-    if (N % q[2]) continue;
+    if (N % q.bn || (q.tile == kTileQ && N == kQkvStride)) continue;
     for (int s = 1; s <= max_splits && s <= 16 && s <= nst; ++s) {
-      const GemmPlan p = make(q[0], q[1], q[2], s);
+      const GemmPlan p = make(q.tile, q.bm, q.bn, s);
       const long long g = (long long)p.m_tiles * p.n_tiles * s;
       if (s > 1 && g > 256) break;
-      const float step = q[0] == kTileL ? 1.29f : q[0] == kTileH ? 0.78f : p.m_tiles == 1 ? 0.75f : 0.45f;
+      const float step = q.tile == kTileM && p.m_tiles == 1 ? 0.75f : s > 1 ? q.split_step : q.step;
       consider(p, 2.4f + (float)((g + 255) / 256) * ((float)((nst + s - 1) / s) * step + 5.f));
     }
   }
@@ -1339,6 +1354,8 @@ static void gemm_launch_main(const GemmArgs& a, const GemmPlan& p, bool f32, boo
                              hipStream_t st) {
   switch (p.tile) {
     case kTileL: launch_gemm<TileL>(a, f32, st); break;
+    case kTileP: launch_gemm<TileP>(a, f32, st); break;
+    case kTileQ: launch_gemm<TileQ>(a, f32, st); break;
     case kTileH: launch_gemm<TileH>(a, f32, st); break;
     case kTileM: launch_gemm<TileM>(a, f32, st); break;
     case kTileS: launch_gemm<TileS>(a, f32, st); break;
@@ -1364,6 +1381,8 @@ int gemm_launch_partials(const void* x, int64_t ldx, const void* w, int64_t ldw,
     a.app = app;
     if (p.tile == kTileL)
       launch_append<TileL>(a, st);
+    else if (p.tile == kTileP)
+      launch_append<TileP>(a, st);
     else if (p.tile == kTileH)
       launch_append<TileH>(a, st);
     else
@@ -1427,6 +1446,8 @@ extern "C" int fqa_gemm_argmax(const void* x, int64_t ldx, const void* w, int64_
   hipStream_t st = (hipStream_t)stream;
   switch (p.tile) {
     case kTileL: launch_argmax<TileL>(a, st); break;
+    case kTileP: launch_argmax<TileP>(a, st); break;
+    case kTileQ: launch_argmax<TileQ>(a, st); break;
     case kTileH: launch_argmax<TileH>(a, st); break;
     case kTileM: launch_argmax<TileM>(a, st); break;
     case kTileS: launch_argmax<TileS>(a, st); break;

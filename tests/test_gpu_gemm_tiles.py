@@ -19,6 +19,11 @@ from tests.test_gpu_gemm import _run_case
     (1100, 256, 1024, {}),                  # split K (partials)
     (1100, 256, 1024, {"out_f32": True}),
     (2300, 2304, 128, {"ldx_pad": 8}),      # several tiles per workgroup slot
+    (384, 24576, 64, {}),                   # 192 x 256 tiles, full rows
+    (300, 24576, 128, {"ldy_pad": 4}),      # ... ragged
+    (500, 24576, 192, {}),                  # 256 x 192 tiles
+    (400, 24576, 64, {"out_f32": True}),
+    (1500, 4096, 12288, {}),                # 192 x 256 with K split
 ])
 def test_gemm_256_tile(gpu, M, N, K, kw):
     _run_case(gpu, M, N, K, seed=M + K, **kw)
@@ -92,6 +97,7 @@ def test_gemm_smaller_workspace(gpu):
     (345, 1024, 0, None),   # 128 x 128 tiles
     (450, 1024, 1, 440),    # ... with the row count inside the last one
     (700, 512, 1, 690),     # 256 x 128 tiles
+    (1500, 256, 0, 1490),   # 192 x 256 tiles
 ])
 def test_qkv_fused_tiles(gpu, M, K, write_k, rows):
     from tests.test_gpu_qkv_fused import _case

@@ -14,6 +14,11 @@ __device__ __forceinline__ void unpack4(uint2 v, float* f) {
   f[3] = __uint_as_float(v.y & 0xffff0000u);
 }
 
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xf, 0xf, true));
+}
+
 // HeadNormRopeKernel's math (engine/src/kernels.cu:97-131) for one head of one row, held
 // by a 16-lane group: lane j of the group holds dims 4j..4j+3 (lo) and 64+4j..64+4j+3 (hi)
 // as packed bf16, so both halves of every rotate-half pair sit in one lane.
@@ -37,8 +42,12 @@ __device__ __forceinline__ void norm_rope_head(uint2 lo, uint2 hi, const float (
     ss = fmaf(x1[e], x1[e], ss);
     ss = fmaf(x2[e], x2[e], ss);
   }
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, kWave);
+  // (lane ^ 1, ^ 2, then ^ 4 and ^ 8 as the mirrors within 8 and 16 lanes, whose quads and
+  // halves already agree: the same sums as xor shuffles, without their LDS round trips)
+  ss += dpp<0xB1>(ss);
+  ss += dpp<0x4E>(ss);
+  ss += dpp<0x141>(ss);
+  ss += dpp<0x140>(ss);
   const float inv = 1.0f / sqrtf(ss / (float)kD + eps);
   float o1[4], o2[4];
 #pragma unroll

@@ -931,6 +931,13 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_slab_kernel(GemmArgs a) {
 //    whole V^T rows (a register transpose of the 16 staged rows); other rows store their
 //    token's column.
 // v is not written to qkv.  Rows at or past meta[FQA_META_ROWS] are not written.
+// What bounds it: latency, with one wave per SIMD.  One head's norm after the other (xor
+// shuffles through LDS in each) and one wave walking all of a V tile's pages cost 12-25 us a
+// tile; with a batch's norms side by side, DPP sums and each wave's rows settled by a lane
+// each, QKV + append with 512-token prompts at 500 / 700 / 1000 / 2048 / 8192 rows 49 / 73 /
+// 76 / 107 / 333 -> 40 / 53 / 57 / 92 / 309 us.  Rows on pages of their own are bound by the
+// CUs that hold V, a lane's 2-byte store per clock (dims in a row; every other dim per store
+// took 1.4 times that): 260 / 500 / 700 / 2048 rows 43 / 52 / 72 / 137 -> 39 / 49 / 63 / 127.
 template <class T>
 __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::Block (&acc)[T::kTM][T::kTN],
                                 int row0, int col0, int wm, int wn, int w, int lane) {
@@ -964,13 +971,15 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::
     const float4 w2 = *reinterpret_cast<const float4*>(wv + 64 + 4 * j);
     const float wa[4] = {w1.x, w1.y, w1.z, w1.w}, wb[4] = {w2.x, w2.y, w2.z, w2.w};
     // (row, head) pairs in batches of kB per lane group: every load of a batch (staged
-    // values, positions, then the cos/sin rows) is issued before any is used
-    constexpr int kB = 8;
+    // values, positions, then the cos/sin rows) is issued before any is used, and the batch's
+    // norms run side by side, before any of its stores: a SIMD has one wave here, so one
+    // head's chain after the other is all latency
     constexpr int kPerGroup = T::kBM * kNH / (T::kWaves * 4);
+    constexpr int kB = kPerGroup / ((kPerGroup + 15) / 16);
     static_assert(kPerGroup % kB == 0, "batches");
     for (int b0 = 0; b0 < kPerGroup; b0 += kB) {
       int rt[kB], pos[kB];
-      uint2 lo[kB], hv[kB];
+      uint2 lo[kB], hv[kB], olo[kB], ohi[kB];
       float4 c4[kB], s4[kB];
 #pragma unroll
       for (int b = 0; b < kB; ++b) {
@@ -990,79 +999,90 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::
       }
 #pragma unroll
       for (int b = 0; b < kB; ++b) {
+        const float cs[4] = {c4[b].x, c4[b].y, c4[b].z, c4[b].w};
+        const float sn[4] = {s4[b].x, s4[b].y, s4[b].z, s4[b].w};
+        norm_rope_head(lo[b], hv[b], wa, wb, cs, sn, p.eps, olo[b], ohi[b]);  // all lanes
+      }
+#pragma unroll
+      for (int b = 0; b < kB; ++b) {
         const int hr = (b0 + b) * T::kWaves * 4 + w * 4 + g;
         const int row = row0 + rt[b], head = head0 + hr % kNH;
         const bool pos_ok = pos[b] >= 0 && pos[b] < p.rope_max_pos;  // false: no such row too
-        const float cs[4] = {c4[b].x, c4[b].y, c4[b].z, c4[b].w};
-        const float sn[4] = {s4[b].x, s4[b].y, s4[b].z, s4[b].w};
-        uint2 olo, ohi;
-        norm_rope_head(lo[b], hv[b], wa, wb, cs, sn, p.eps, olo, ohi);  // all lanes
         if (row >= T_rows) continue;
         if (!pos_ok) {  // no table row: the projection's values, as unfused
-          olo = lo[b];
-          ohi = hv[b];
+          olo[b] = lo[b];
+          ohi[b] = hv[b];
         }
         if (!is_k || p.write_k) {
           uint16_t* d = qkv + (long long)row * a.ldy + head * kD + 4 * j;
-          *reinterpret_cast<uint2*>(d) = olo;
-          *reinterpret_cast<uint2*>(d + 64) = ohi;
+          *reinterpret_cast<uint2*>(d) = olo[b];
+          *reinterpret_cast<uint2*>(d + 64) = ohi[b];
         }
         if (is_k && pos_ok) {
           const int slot = s_slot[rt[b]];
           const long long page = slot / kPage;
           if (slot >= 0 && page < p.pool_pages) {
             uint16_t* kd = p.pool + run_offset(page, head - kHq) + (slot % kPage) * kD + 4 * j;
-            *reinterpret_cast<uint2*>(kd) = olo;
-            *reinterpret_cast<uint2*>(kd + 64) = ohi;
+            *reinterpret_cast<uint2*>(kd) = olo[b];
+            *reinterpret_cast<uint2*>(kd + 64) = ohi[b];
           }
         }
       }
     }
     return;
   }
-  // v heads: one wave per row; lane l holds dims 2l, 2l+1 of each head
-  for (int rt = w; rt < T::kBM; rt += T::kWaves) {
-    const int row = row0 + rt;
-    if (row >= T_rows) break;
-    const int pos = s_pos[rt];
-    if (pos < 0 || pos >= p.rope_max_pos) continue;  // the append skips such rows
-    const int slot = s_slot[rt];
-    const long long page = slot / kPage;
-    if (slot < 0 || page >= p.pool_pages) continue;
-    const int tok = slot % kPage, lt = rt - tok;  // the page's first row, in the tile
-    // A page whose rows all lie in the tile (and that the append kernel would write whole:
-    // same test) is written by its first row; any other row writes its own column.  Both
-    // give the same bytes.
-    bool whole = lt >= 0 && lt + kPage <= T::kBM && row0 + lt + kPage <= T_rows;
-    if (whole)
-      whole = s_slot[lt] == slot - tok && s_slot[lt + kPage - 1] == slot - tok + kPage - 1 &&
-              s_pos[lt] >= 0 && s_pos[lt + kPage - 1] < p.rope_max_pos;
-    if (whole && tok != 0) continue;
+  // v heads.  Each wave takes kBM / 4 rows in a row; lane l first settles row l: skipped,
+  // written as a whole page, or its column.
+  constexpr int kRows = T::kBM / T::kWaves;
+  static_assert(kRows <= kWave && kRows % kPage == 0, "a lane per row");
+  const int rt = w * kRows + min(lane, kRows - 1);
+  const int pos = s_pos[rt], slot = s_slot[rt];
+  const int tok = slot % kPage, lt = rt - tok;  // the page's first row, in the tile
+  // (a row without a position is no row, or one that the append skips)
+  const bool valid = lane < kRows && pos >= 0 && pos < p.rope_max_pos && slot >= 0 &&
+                     slot / kPage < p.pool_pages;
+  // A page whose rows all lie in the tile (and that the append kernel would write whole:
+  // same test) is written by its first row; any other row writes its own column.  Both
+  // give the same bytes.
+  bool whole = valid && lt >= 0 && lt + kPage <= T::kBM && row0 + lt + kPage <= T_rows;
+  if (whole)
+    whole = s_slot[lt] == slot - tok && s_slot[lt + kPage - 1] == slot - tok + kPage - 1 &&
+            s_pos[lt] >= 0 && s_pos[lt + kPage - 1] < p.rope_max_pos;
+  const int kvh0 = head0 - kHq - kHkv;
+  // whole pages: lane l holds dims 2l, 2l+1 of each head
+  for (uint64_t m = __ballot(whole && tok == 0); m; m &= m - 1) {
+    const int l = __ffsll((unsigned long long)m) - 1, r = w * kRows + l;
+    const long long page = __builtin_amdgcn_readlane(slot, l) / kPage;
 #pragma unroll
     for (int hi = 0; hi < kNH; ++hi) {
-      const int kvh = head0 + hi - kHq - kHkv;
-      uint16_t* vt = p.pool + run_offset(page, kvh) + kVOff + 2 * lane * kPage;
-      if (whole) {
-        uint32_t x[kPage];
+      uint16_t* vt = p.pool + run_offset(page, kvh0 + hi) + kVOff + 2 * lane * kPage;
+      uint32_t x[kPage];
 #pragma unroll
-        for (int t = 0; t < kPage; ++t)
-          x[t] = *reinterpret_cast<const uint32_t*>(lds + (rt + t) * kTP + (hi * kD + 2 * lane) * 2);
-        uint32_t y0[8], y1[8];
+      for (int t = 0; t < kPage; ++t)
+        x[t] = *reinterpret_cast<const uint32_t*>(lds + (r + t) * kTP + (hi * kD + 2 * lane) * 2);
+      uint32_t y0[8], y1[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          y0[k] = __builtin_amdgcn_perm(x[2 * k + 1], x[2 * k], 0x05040100u);
-          y1[k] = __builtin_amdgcn_perm(x[2 * k + 1], x[2 * k], 0x07060302u);
-        }
-        uint4* v4 = reinterpret_cast<uint4*>(vt);
-        v4[0] = make_uint4(y0[0], y0[1], y0[2], y0[3]);
-        v4[1] = make_uint4(y0[4], y0[5], y0[6], y0[7]);
-        v4[2] = make_uint4(y1[0], y1[1], y1[2], y1[3]);
-        v4[3] = make_uint4(y1[4], y1[5], y1[6], y1[7]);
-      } else {
-        const uint32_t x = *reinterpret_cast<const uint32_t*>(lds + rt * kTP + (hi * kD + 2 * lane) * 2);
-        vt[tok] = (uint16_t)x;
-        vt[kPage + tok] = (uint16_t)(x >> 16);
+      for (int k = 0; k < 8; ++k) {
+        y0[k] = __builtin_amdgcn_perm(x[2 * k + 1], x[2 * k], 0x05040100u);
+        y1[k] = __builtin_amdgcn_perm(x[2 * k + 1], x[2 * k], 0x07060302u);
       }
+      uint4* v4 = reinterpret_cast<uint4*>(vt);
+      v4[0] = make_uint4(y0[0], y0[1], y0[2], y0[3]);
+      v4[1] = make_uint4(y0[4], y0[5], y0[6], y0[7]);
+      v4[2] = make_uint4(y1[0], y1[1], y1[2], y1[3]);
+      v4[3] = make_uint4(y1[4], y1[5], y1[6], y1[7]);
+    }
+  }
+  for (uint64_t m = __ballot(valid && !whole); m; m &= m - 1) {
+    const int l = __ffsll((unsigned long long)m) - 1, r = w * kRows + l;
+    const int sl = __builtin_amdgcn_readlane(slot, l);
+    // here lane l holds dims l and 64 + l: a store's 64 places lie in 2 KiB in a row
+#pragma unroll
+    for (int hi = 0; hi < kNH; ++hi) {
+      const uint16_t* x = reinterpret_cast<const uint16_t*>(lds + r * kTP) + hi * kD + lane;
+      uint16_t* vt = p.pool + run_offset(sl / kPage, kvh0 + hi) + kVOff + lane * kPage + sl % kPage;
+      vt[0] = x[0];
+      vt[kWave * kPage] = x[kWave];
     }
   }
 }

@@ -1224,6 +1224,12 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
   };
   if (M <= 128 && N / 128 >= 160)
     return M > 64 ? make(kTileM, 128, 128, 1) : M > 32 ? make(kTileS, 64, 128, 1) : make(kTileT, 32, 128, 1);
+  // the QKV width at 449..512 rows (where the call may split): the append kernel reads two
+  // planes.  With the append in the epilogue of 128 x 128 tiles, rows on their own pages keep
+  // the few CUs that hold V busy after all others: QKV + append at 450 / 500 / 512 such rows
+  // 43.3 / 49.4 / 49.4 us, split 42.4 / 43.9 / 44.2; 512-token prompts 36.4 / 40.4 / 41.2, split
+  // 42.1 / 42.8 / 43.1.  At 448 own-page rows the epilogue takes 43.1, at 260 / 400 39 / 40.
+  if (N == kQkvStride && M > 448 && M <= 512 && max_splits > 1) return make(kTileH, 256, 128, 2);
   GemmPlan best{};
   float best_us = 3.4e38f;
   auto consider = [&](const GemmPlan& p, float us) {

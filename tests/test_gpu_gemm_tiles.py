@@ -95,7 +95,8 @@ def test_gemm_smaller_workspace(gpu):
     (100, 64, 1, None),     # one k step: the 128-row tile's append epilogue
     (129, 1024, 0, None),   # a slab's fp32 sums through the append kernel
     (345, 1024, 0, None),   # 128 x 128 tiles
-    (450, 1024, 1, 440),    # ... with the row count inside the last one
+    (448, 1024, 1, 440),    # ... with the row count inside the last one
+    (450, 1024, 1, 440),    # two planes of 256 x 128 tiles through the append kernel
     (700, 512, 1, 690),     # 256 x 128 tiles
     (1500, 256, 0, 1490),   # 192 x 256 tiles
 ])

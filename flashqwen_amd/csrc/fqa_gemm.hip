@@ -23,6 +23,7 @@
 #include "fqa_append_math.h"
 #include "fqa_common.h"
 #include "fqa_gemm_internal.h"
+#include "fqa_quad_schedule.h"
 
 #include <type_traits>
 
@@ -66,39 +67,10 @@ struct Tile {
     return (wn * kTN + cb) * 32 + 8 * q + 4 * (lane >> 5);
   }
 };
-// The tiles of gemm_quad_kernel: 4 waves, 2 x 2.  Each operand tile is two halves (rows
-// 0 .. kBM/2 - 1 and the rest; W rows likewise) and a wave's kBM/2 x kBN/2 outputs are four
-// quadrants, one per (x half, W half), of kQM x kQN 16 x 16 blocks.
-template <int kBM_, int kBN_, int kRing_>
-struct Quad {
-  static constexpr int kBM = kBM_, kBN = kBN_, kRing = kRing_;
-  static constexpr int kWM = 2, kWN = 2, kQM = kBM / 64, kQN = kBN / 64;
-  static constexpr int kTM = 2 * kQM, kTN = 2 * kQN;
-  static constexpr int kBK = 64, kPitch = 128;
-  static constexpr int kHalfA = kBM / 2 * kPitch, kHalfB = kBN / 2 * kPitch;  // bytes per step
-  static constexpr int kStage = 2 * (kHalfA + kHalfB);
-  static constexpr int kWaves = 4, kThreads = 256;
-  static constexpr int kDmaA = kBM / 64, kDmaB = kBN / 64;  // DMA instructions per wave per half
-  static_assert(kRing >= 2 && kRing * kStage <= 160 * 1024, "LDS");
-  __device__ static int swz(int r) { return (r >> 1) & 7; }
-  typedef float4_t Block;
-  static constexpr int kQuads = 1, kRowLanes = 16;
-  __device__ static int row(int wm, int rb, int lane) {
-    return (rb / kQM) * (kBM / 2) + wm * (kBM / 4) + (rb % kQM) * 16 + (lane & 15);
-  }
-  __device__ static int col(int wn, int cb, int, int lane) {
-    return (cb / kQN) * (kBN / 2) + wn * (kBN / 4) + (cb % kQN) * 16 + 4 * (lane >> 4);
-  }
-};
 template <class T>
 constexpr bool kIsQuad = false;
 template <int M, int N, int R>
 constexpr bool kIsQuad<Quad<M, N, R>> = true;
-using TileL = Quad<256, 256, 2>;
-using TileP = Quad<192, 256, 2>;
-using TileQ = Quad<256, 192, 2>;
-using TileH = Quad<256, 128, 3>;
-using TileM = Quad<128, 128, 5>;
 using TileS = Tile<1, 4, 2, 1, 6>;  // 64 x 128
 using TileT = Tile<1, 4, 1, 1, 8>;  // 32 x 128: a few decode rows
 
@@ -510,20 +482,8 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
   tile_epilogue<T, kF32Out, false, kArgmax, false>(a, lds, acc, row0, col0, tn, sp, wm, wn, w, lane);
 }
 
-// The large tiles: one wave per SIMD, each a quarter of the tile (128 x 128 of 256 x 256).  A
-// step is 64 k of both operands, four halves (x rows: A0, A1; W rows: B0, B1), kRing steps in
-// LDS, and four phases per wave, one per quadrant, in the order (A0,B0) (A0,B1) (A1,B1)
-// (A1,B0).
-//  * Every phase reads from LDS the half the next phase adds (B1, A1, A0(t+1), B0(t+1)), and
-//    issues the DMA of one half (A1(t+R-1), A0(t+R), B0(t+R), B1(t+R), R = kRing), spread
-//    between its MFMAs, so no wait sits in front of an MFMA and a half has 3 phases or more
-//    to land.
-//  * Two barriers per step, each behind a vmcnt that leaves the newest halves in flight:
-//    after phase 2 A0(t+1) and B0(t+1) are in LDS for every wave, after phase 4 B1(t+1) and
-//    A1(t+1).  A half's slot is refilled only after a barrier that follows every wave's last
-//    use of it: fragments are consumed by MFMAs before the barrier, except A0(t+1)'s, which
-//    the lgkmcnt before the second barrier waits for (B0(t+1)'s are newer; they are consumed
-//    in phase 1 of t+1, a barrier before B0's refill).
+// The large tiles: one wave per SIMD, each a quarter of the tile (128 x 128 of 256 x 256), its
+// steps in the order of QuadSchedule.
 //  * What bounds the 256 x 256 tile: the MFMAs at the clock the card holds under them (taking
 //    all DMA out of the loop changes 289 us to 292 on 8192 x 6144 x 4096, all waits and
 //    barriers to 282), then ~5 us per tile to start and to store.  16 x 16 x 32 MFMAs beat
@@ -534,9 +494,78 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_kernel(GemmArgs a) {
 //    1.42-1.51 PFLOP/s.  256 x 128 and 128 x 128 against their 8- and 4-wave predecessors:
 //    qkv at 1000 rows 61 -> 52 us, o_proj at 700 rows 39 -> 33, gate_up at 512 rows (256 x
 //    256) 122 -> 94, down at 700 rows (256 x 256, K split 5 ways) 93 -> 74.
+// QuadSchedule's operations, for one wave.  LDS: the x halves of slot b at b * 2 kHalfA, the
+// W halves at kB + b * 2 kHalfB.
+template <class T, bool kNT>
+struct QuadOps {
+  static constexpr int kQM = T::kQM, kQN = T::kQN, kB = T::kRing * 2 * T::kHalfA;
+  char* lds;
+  uint32_t dst_a, dst_b;  // this wave's share of a half, in slot 0
+  uint32_t off_a[2][T::kDmaA], off_b[2][T::kDmaB];
+  // where the newest staged step starts (past the end the last step is staged again, never
+  // read, so that every wait count holds), and the x of the step before it
+  const uint16_t *xs, *ws, *xs_prev;
+  int n, pos;  // steps; the one that xs and ws point at
+  long long kstride;
+  int pa[2], pb[2];
+  bf16x8 af[2][kQM][2], bf[2][kQN][2];  // [half][r][kk]
+  float4_t acc[T::kTM][T::kTN];
+
+  __device__ __forceinline__ void stage_a(int h, int slot, int i) {
+    dma16(xs, off_a[h][i], dst_a + (2 * slot + h) * T::kHalfA + i * 1024);
+  }
+  __device__ __forceinline__ void stage_a1_prev(int slot, int i) {
+    dma16(xs_prev, off_a[1][i], dst_a + (2 * slot + 1) * T::kHalfA + i * 1024);
+  }
+  __device__ __forceinline__ void stage_b(int h, int slot, int i) {
+    dma16_w<kNT>(ws, off_b[h][i], dst_b + (2 * slot + h) * T::kHalfB + i * 1024);
+  }
+  __device__ __forceinline__ void keep() { xs_prev = xs; }
+  __device__ __forceinline__ void advance(bool more) {
+    if (!more) return;
+    const long long d = ++pos == n ? kstride - n * kstride : kstride;
+    pos = pos == n ? 0 : pos;
+    xs += d;
+    ws += d;
+  }
+  // fragment f = kk * (blocks) + r of half h, in the slot that pa / pb point at
+  __device__ __forceinline__ void read_a(int h, int f) {
+    af[h][f % kQM][f / kQM] = *reinterpret_cast<const bf16x8*>(
+        lds + pa[f / kQM] + h * T::kHalfA + (f % kQM) * 16 * T::kPitch);
+  }
+  __device__ __forceinline__ void read_b(int h, int f) {
+    bf[h][f % kQN][f / kQN] = *reinterpret_cast<const bf16x8*>(
+        lds + pb[f / kQN] + h * T::kHalfB + (f % kQN) * 16 * T::kPitch);
+  }
+  __device__ __forceinline__ void turn(int dslot) {
+    const int da = dslot * 2 * T::kHalfA, db = dslot * 2 * T::kHalfB;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      pa[kk] += da;
+      pb[kk] += db;
+    }
+  }
+  __device__ __forceinline__ void mfma(int i, int j, int r, int c, int kk) {
+    acc[kQM * i + r][kQN * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+        bf[j][c][kk], af[i][r][kk], acc[kQM * i + r][kQN * j + c], 0, 0, 0);
+  }
+  template <int N>
+  __device__ __forceinline__ void wait_vm() {
+    fqa::wait_vm<N>();
+  }
+  template <int N>
+  __device__ __forceinline__ void wait_lgkm() {
+    static_assert(N >= 0 && N < 16, "lgkmcnt");
+    __builtin_amdgcn_s_waitcnt(0xC07F | N << 8);
+  }
+  __device__ __forceinline__ void barrier() { fqa::barrier(); }
+  __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+};
+
 template <class T, bool kNT, bool kF32Out, bool kPartial, bool kArgmax = false, bool kAppend = false>
 __global__ void __launch_bounds__(T::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
-  constexpr int kRing = T::kRing, kQM = T::kQM, kQN = T::kQN, dA = T::kDmaA, dB = T::kDmaB;
+  constexpr int dA = T::kDmaA, dB = T::kDmaB;
+  using Ops = QuadOps<T, kNT>;
   __shared__ __attribute__((aligned(1024))) char lds[kGemmLds<T, kAppend>];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -547,169 +576,55 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
   const int row0 = tm * T::kBM, col0 = tn * T::kBN;
   const int nst = a.K / T::kBK;
   const int n = (nst - sp + a.splits - 1) / a.splits;  // >= 1: splits <= steps
-  const long long kstride = (long long)a.splits * T::kBK;
+  Ops o;
+  o.lds = lds;
+  o.n = n;
+  o.kstride = (long long)a.splits * T::kBK;
 
-  // LDS: the x halves of slot b at b * 2 kHalfA, the W halves at kB + b * 2 kHalfB.
   // Wave w's DMA instruction i of a half covers rows 8 (w d + i) + lane / 8 (d instructions
   // per wave); a lane fills LDS chunk lane % 8 of its row, so it reads global chunk
   // (lane % 8) ^ swz(row).
-  constexpr int kB = kRing * 2 * T::kHalfA;
-  uint32_t off_a[2][dA], off_b[2][dB];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int i = 0; i < dA; ++i) {
       const int r = 8 * (w * dA + i) + (lane >> 3);
       const int gr = min(row0 + T::kBM / 2 * h + r, a.M - 1);
-      off_a[h][i] = (uint32_t)((long long)gr * a.ldx * 2) + ((lane & 7) ^ T::swz(r)) * 16;
+      o.off_a[h][i] = (uint32_t)((long long)gr * a.ldx * 2) + ((lane & 7) ^ T::swz(r)) * 16;
     }
 #pragma unroll
     for (int i = 0; i < dB; ++i) {
       const int r = 8 * (w * dB + i) + (lane >> 3);
-      off_b[h][i] = (uint32_t)((long long)(col0 + T::kBN / 2 * h + r) * a.ldw * 2) +
-                    ((lane & 7) ^ T::swz(r)) * 16;
+      o.off_b[h][i] = (uint32_t)((long long)(col0 + T::kBN / 2 * h + r) * a.ldw * 2) +
+                      ((lane & 7) ^ T::swz(r)) * 16;
     }
   }
-  const uint32_t dst_a = lds_base + w * (dA * 1024), dst_b = lds_base + kB + w * (dB * 1024);
-  auto stage_a = [&](const uint16_t* xs, int h, int slot, int i) {
-    dma16(xs, off_a[h][i], dst_a + (2 * slot + h) * T::kHalfA + i * 1024);
-  };
-  auto stage_b = [&](const uint16_t* ws, int h, int slot, int i) {
-    dma16_w<kNT>(ws, off_b[h][i], dst_b + (2 * slot + h) * T::kHalfB + i * 1024);
-  };
-  // xs, ws: where the newest staged step starts; past the end the last step is staged again
-  // (never read), so that every wait count holds.  xs_prev: the step before it.
-  const uint16_t* xs = a.x + (long long)sp * T::kBK;
-  const uint16_t* ws = a.w + (long long)sp * T::kBK;
+  o.dst_a = lds_base + w * (dA * 1024);
+  o.dst_b = lds_base + Ops::kB + w * (dB * 1024);
   // one row tile, unsplit, up to 128 rows: W streams from HBM
   constexpr bool kSeg = kNT && T::kBM == 128;
   const Segments segs{n, kSeg ? (int)(blockIdx.x >> 3) & 3 : 0};
-  int pos = segs.first();
-  xs += pos * kstride;
-  ws += pos * kstride;
-  auto advance = [&](bool more) {
-    if (!more) return;
-    const long long d = ++pos == n ? kstride - n * kstride : kstride;
-    pos = pos == n ? 0 : pos;
-    xs += d;
-    ws += d;
-  };
-  const uint16_t* xs_prev = xs;
-#pragma unroll
-  for (int b = 0; b < kRing; ++b) {  // every slot but A1 of the last
-#pragma unroll
-    for (int i = 0; i < dA; ++i) stage_a(xs, 0, b, i);
-#pragma unroll
-    for (int i = 0; i < dB; ++i) stage_b(ws, 0, b, i);
-#pragma unroll
-    for (int i = 0; i < dB; ++i) stage_b(ws, 1, b, i);
-    xs_prev = xs;
-    if (b + 1 < kRing) {
-#pragma unroll
-      for (int i = 0; i < dA; ++i) stage_a(xs, 1, b, i);
-      advance(b + 1 < n);
-    }
-  }
+  o.pos = segs.first();
+  o.xs = a.x + (long long)sp * T::kBK + o.pos * o.kstride;
+  o.ws = a.w + (long long)sp * T::kBK + o.pos * o.kstride;
+  QuadSchedule<T> schedule;
+  schedule.stage_first(o, n);
 
   // fragment (r, kk) of a half: row (wave's first) + 16 r + lane % 16, 16-byte chunk
   // 4 kk + lane / 16
-  int pa[2], pb[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     const int c = ((4 * kk + (lane >> 4)) ^ T::swz(lane & 15)) * 16;
-    pa[kk] = (wm * (T::kBM / 4) + (lane & 15)) * T::kPitch + c;
-    pb[kk] = kB + (wn * (T::kBN / 4) + (lane & 15)) * T::kPitch + c;
+    o.pa[kk] = (wm * (T::kBM / 4) + (lane & 15)) * T::kPitch + c;
+    o.pb[kk] = Ops::kB + (wn * (T::kBN / 4) + (lane & 15)) * T::kPitch + c;
   }
-  bf16x8 af[2][kQM][2], bf[2][kQN][2];  // [half][r][kk]
-  // fragment f = kk * (blocks) + r of half h, in the slot that pa / pb point at
-  auto read_a = [&](int h, int f) {
-    af[h][f % kQM][f / kQM] = *reinterpret_cast<const bf16x8*>(
-        lds + pa[f / kQM] + h * T::kHalfA + (f % kQM) * 16 * T::kPitch);
-  };
-  auto read_b = [&](int h, int f) {
-    bf[h][f % kQN][f / kQN] = *reinterpret_cast<const bf16x8*>(
-        lds + pb[f / kQN] + h * T::kHalfB + (f % kQN) * 16 * T::kPitch);
-  };
-  float4_t acc[T::kTM][T::kTN];
+  auto& acc = o.acc;
 #pragma unroll
   for (int rb = 0; rb < T::kTM; ++rb)
 #pragma unroll
     for (int cb = 0; cb < T::kTN; ++cb) acc[rb][cb] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  // One phase: the MFMAs of quadrant (x half i, W half j), kk outermost; between(q) places
-  // fragment reads and DMA instructions after MFMA q.
-  constexpr int kN = 2 * kQM * kQN;
-  auto phase = [&](int i, int j, auto&& between) {
-#pragma unroll
-    for (int q = 0; q < kN; ++q) {
-      const int kk = q / (kQM * kQN), r = q / kQN % kQM, c = q % kQN;
-      acc[kQM * i + r][kQN * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          bf[j][c][kk], af[i][r][kk], acc[kQM * i + r][kQN * j + c], 0, 0, 0);
-      between(q);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  // after MFMA q: those of `count` reads spread over the phase's first half, of `count` DMA
-  // instructions spread over all of it
-  auto reads = [&](int q, int count, auto&& f) {
-#pragma unroll
-    for (int e = 0; e < count; ++e)
-      if (((2 * e + 1) * (kN / 2)) / (2 * count) == q) f(e);
-  };
-  auto stages = [&](int q, int count, auto&& f) {
-#pragma unroll
-    for (int e = 0; e < count; ++e)
-      if (((2 * e + 1) * kN) / (2 * count) == q) f(e);
-  };
-  wait_vm<2 * dB + dA + (kRing - 2) * 2 * (dA + dB)>();  // step 0
-  barrier();
-#pragma unroll
-  for (int f = 0; f < 2 * kQM; ++f) read_a(0, f);
-#pragma unroll
-  for (int f = 0; f < 2 * kQN; ++f) read_b(0, f);
-  int cur = 0;  // step t's slot
-  int t = 0;
-  auto steps = [&](int end) {
-    for (; t < end; ++t) {
-      const int prev = cur == 0 ? kRing - 1 : cur - 1;
-      const bool more = t + kRing < n;
-      advance(more);
-      phase(0, 0, [&](int q) {
-        reads(q, 2 * kQN, [&](int f) { read_b(1, f); });
-        stages(q, dA, [&](int i) { stage_a(xs_prev, 1, prev, i); });  // A1(t + kRing - 1)
-      });
-      phase(0, 1, [&](int q) {
-        reads(q, 2 * kQM, [&](int f) { read_a(1, f); });
-        stages(q, dA, [&](int i) { stage_a(xs, 0, cur, i); });  // A0(t + kRing)
-      });
-      wait_vm<dB + 2 * dA + (kRing - 2) * 2 * (dA + dB)>();  // A0(t+1), B0(t+1)
-      barrier();
-      const int dslot = cur == kRing - 1 ? 1 - kRing : 1;  // to step t + 1's slot
-      const int da = dslot * 2 * T::kHalfA, db = dslot * 2 * T::kHalfB;
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        pa[kk] += da;
-        pb[kk] += db;
-      }
-      phase(1, 1, [&](int q) {
-        reads(q, 2 * kQM, [&](int f) { read_a(0, f); });
-        stages(q, dB, [&](int i) { stage_b(ws, 0, cur, i); });  // B0(t + kRing)
-      });
-      phase(1, 0, [&](int q) {  // B0(t+1)'s fragments as B0(t)'s are used up
-        if (q >= kN / 2 && q < kN / 2 + kQN) read_b(0, q - kN / 2);
-        if (q == kN - 1)
-#pragma unroll
-          for (int f = kQN; f < 2 * kQN; ++f) read_b(0, f);
-        stages(q, dB, [&](int i) { stage_b(ws, 1, cur, i); });  // B1(t + kRing)
-      });
-      wait_vm<2 * dB + dA + (kRing - 2) * 2 * (dA + dB)>();  // B1(t+1), A1(t+1)
-      // lgkmcnt(2 kQN): A0(t+1) is read (B0's are newer)
-      __builtin_amdgcn_s_waitcnt(0xC07F | (2 * kQN) << 8);
-      barrier();
-      xs_prev = xs;
-      cur = cur == kRing - 1 ? 0 : cur + 1;
-    }
-  };
+  schedule.read_first(o);
+  auto steps = [&](int end) { schedule.steps(o, n, end); };
   if constexpr (kSeg)
     run_segments(segs, acc, steps);
   else

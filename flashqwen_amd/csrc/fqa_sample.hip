@@ -15,8 +15,8 @@
 // the exact smallest kept weight after 3 levels, and with it each wave's kept mass.  A top-p
 // row is read 3 times in full (max + sum, level 1, and a pass that copies the weights of the
 // boundary bin into LDS, on which levels 2 and 3 run).  Only when the boundary bin may hold
-// more than 16384 weights is the row read a 4th time for level 3, and once more where the
-// boundary lies below 2^-31 of the largest weight.  A temperature-only row is read once (its
+// more than 16384 weights (copy_fits) is the row read a 4th time for level 3, and once more
+// where the boundary lies below 2^-31 of the largest weight.  A temperature-only row is read once (its
 // kept mass per wave is the rescaled pass-1 sum); the pick then reads 1/16 of one wave's
 // segment.
 //
@@ -30,6 +30,7 @@
 // top-p 0.9 71 -> 61, nearly flat rows 185 -> 76; 256 rows: 32.7 -> 32.0, 37.4 -> 36.6, 93 ->
 // 93 (HBM and the caches carry the reads there), 207 -> 115.
 #include "fqa_common.h"
+#include "fqa_sample_select.h"
 
 #include <cfloat>
 
@@ -42,18 +43,6 @@ constexpr int kBins = 2048;  // histogram bins per radix level (levels use 11, 1
 constexpr int kChunk = 4;    // 256-element steps whose loads a wave issues back to back
 constexpr int kCols = 256;   // level-1 bins with a column per lane: the 31 octaves below 1
 constexpr int kCol0 = (127 << 3) + 8 - kCols;  // ... from this bin on (bits 30..20)
-constexpr int kCandCap = 16384;  // boundary-bin weights that the LDS copy holds
-// Histogram masses are exact integers: a weight with exponent field E adds its 24-bit
-// significand, and a bin's mass is that sum times 2^(max(E, 1) - 150) (every bin holds one
-// exponent).  ds_add_u64 runs at several times the rate of ds_add_f32 on gfx950, whose
-// float adds were most of a top-p row's time; the sums also no longer depend on the order
-// the atomics land in, so the kept set is the same on every run.
-__device__ __forceinline__ unsigned long long significand(uint32_t bits) {
-  return (bits & 0x7fffffu) | (bits >= 0x800000u ? 0x800000u : 0u);
-}
-__device__ __forceinline__ float bin_mass(unsigned long long sum, int exp_field) {
-  return ldexpf((float)sum, max(exp_field, 1) - 150);
-}
 
 struct SampArgs {
   const float* logits;
@@ -342,8 +331,7 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
       b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
     }
     const int e1 = b1 >> 3;  // the exponent field of every weight in bin b1
-    // A normal weight's significand is 2^23 or more, so this bin's weights fit the copy.
-    const bool copy = e1 > 0 && (hcnt[b1] >> 23) <= kCandCap;
+    const bool copy = copy_fits(hcnt[b1], b1, x_min);
     // pass 3: per lane, the mass of the weights above bin b1 (all kept), and the weights in
     // bin b1 copied into LDS (low 20 bits and the wave), on which level 2 (bits 19..9),
     // level 3 and the kept masses run without reading the row again; or level 2 here.

@@ -65,3 +65,21 @@ def test_rows_on_four_bytes(gpu):
         got = sample(x, *(torch.from_numpy(v).to(gpu) for v in (it, tp, u)))
         assert np.array_equal(got.cpu().numpy(), want)
         wide.fill_(99.0)
+
+
+@pytest.mark.gpu
+def test_bin_cut_by_the_smallest_counted_weight(gpu):
+    """top_p so close to 1 that the boundary bin is the one the smallest counted weight cuts:
+    more of its weights lie in the bin than its histogram counts (tests/test_sample_select.py),
+    and the row is read again instead of copied."""
+    from tests.test_sample_select import close_to_one, cut_bin_row
+
+    tp = close_to_one()
+    lg = np.tile(cut_bin_row(), (len(tp), 1))
+    rng = np.random.default_rng(9)
+    it, u = np.ones(len(tp), np.float32), rng.random(len(tp)).astype(np.float32)
+    got = _run(lg, it, tp, u)
+    # equal weights side by side: a draw within fp32 rounding of the total (1e-5 of 150000
+    # tokens) falls on a neighbour, which _check_sampled allows
+    _check_sampled(lg, it, tp, u, got)
+    assert np.array_equal(_run(lg, it, tp, u), got)

@@ -41,8 +41,6 @@ constexpr int kSThreads = 1024;
 constexpr int kSWaves = kSThreads / kWave;
 constexpr int kBins = 2048;  // histogram bins per radix level (levels use 11, 11, 9 bits)
 constexpr int kChunk = 4;    // 256-element steps whose loads a wave issues back to back
-constexpr int kCols = 256;   // level-1 bins with a column per lane: the 31 octaves below 1
-constexpr int kCol0 = (127 << 3) + 8 - kCols;  // ... from this bin on (bits 30..20)
 
 struct SampArgs {
   const float* logits;
@@ -290,9 +288,8 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint32_t bits = __float_as_uint(weight(x[u][e]));
-          const int b = (int)(bits >> 20) - kCol0;
-          if (b >= 0 && __uint_as_float(bits) >= x_min)
-            atomicAdd(&big[b * kWave + lane], significand(bits));
+          if (in_columns(bits, x_min))
+            atomicAdd(&big[((bits >> 20) - kCol0) * kWave + lane], significand(bits));
         }
     });
     __syncthreads();

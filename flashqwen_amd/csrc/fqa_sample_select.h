@@ -19,6 +19,16 @@ __host__ __device__ inline float bin_mass(unsigned long long sum, int exp_field)
   return ldexpf((float)sum, (exp_field > 1 ? exp_field : 1) - 150);
 }
 
+constexpr int kCols = 256;  // level-1 bins with a column per lane: the 31 octaves below 1
+constexpr int kCol0 = (127 << 3) + 8 - kCols;  // ... from this bin on (bits 30..20)
+
+// Whether a weight is counted in a column.  A NaN (of a NaN or infinite logit) has a bin past
+// the columns, and compiled without NaN semantics the comparison with x_min may let it pass.
+__host__ __device__ inline bool in_columns(uint32_t bits, float x_min) {
+  return bits - ((uint32_t)kCol0 << 20) < ((uint32_t)kCols << 20) &&
+         __builtin_bit_cast(float, bits) >= x_min;
+}
+
 constexpr int kCandCap = 16384;  // boundary-bin weights that the LDS copy holds
 
 // Whether every weight in level-1 bin `bin` (bits 30..20) fits the LDS copy, `sum` being the

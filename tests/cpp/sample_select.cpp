@@ -8,11 +8,16 @@
 //
 // prints one line per top_p: "bin x_min_bin counted in_bin fits", `counted` being the most
 // weights that the bin's histogram allows for and `in_bin` what pass 3 copies.
+//
+//   sample_select columns
+//
+// checks that every weight counted in a column (in_columns) has one, whatever its bits.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <string>
 #include <vector>
 
 #include "../../flashqwen_amd/csrc/fqa_sample_select.h"
@@ -67,9 +72,27 @@ void pass1(const std::vector<float>& x, float& m, float& Z) {
     }
   }
 }
+
+int check_columns() {
+  const uint32_t nan = 0x7fc00000u;
+  for (float x_min : {0.f, 1e-9f, 0.5f, __builtin_bit_cast(float, nan)})
+    for (uint32_t bin = 0; bin < 4096; ++bin)
+      for (uint32_t low : {0u, 1u, 0xfffffu}) {
+        const uint32_t bits = bin << 20 | low;
+        const int col = (int)bin - kCol0;
+        const bool in = in_columns(bits, x_min);
+        if (in && (col < 0 || col >= kCols)) {
+          std::printf("weight bits %08x, x_min %g: column %d\n", bits, x_min, col);
+          return 1;
+        }
+        if (x_min == 0.f && in != (col >= 0 && col < kCols)) return 1;
+      }
+  return 0;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
+  if (std::string(argv[1]) == "columns") return check_columns();
   const int N = std::atoi(argv[1]);
   std::vector<float> x(N);
   if (std::fread(x.data(), 4, N, stdin) != (size_t)N) return 2;

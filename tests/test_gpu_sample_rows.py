@@ -83,3 +83,29 @@ def test_bin_cut_by_the_smallest_counted_weight(gpu):
     # tokens) falls on a neighbour, which _check_sampled allows
     _check_sampled(lg, it, tp, u, got)
     assert np.array_equal(_run(lg, it, tp, u), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [1025, 151936])
+def test_rows_with_nan_and_inf(gpu, vocab):
+    """Rows with NaN or infinite logits give some token of the vocabulary and leave the rows
+    beside them alone."""
+    rng = np.random.default_rng(vocab + 1)
+    B = 16
+    lg = _rows(rng, B, vocab)
+    it = np.where(np.arange(B) % 5 == 4, 0.0, 1.0).astype(np.float32)
+    tp = rng.choice([1.0, 0.95, 0.5], size=B).astype(np.float32)
+    tp[:8:2] = 0.9
+    u = rng.random(B).astype(np.float32)
+    want = _run(lg, it, tp, u)
+    bad = lg.copy()
+    bad[0, vocab // 2] = np.nan
+    bad[2, [3, vocab // 3]] = np.inf
+    bad[4, :] = np.nan
+    bad[6, :] = np.inf
+    bad[8, ::3] = np.nan
+    bad[9, 7] = np.nan
+    got = _run(bad, it, tp, u)
+    assert np.all((got >= 0) & (got < vocab))
+    ordinary = [b for b in range(B) if b not in (0, 2, 4, 6, 8, 9)]
+    assert np.array_equal(got[ordinary], want[ordinary])

@@ -1,7 +1,8 @@
-"""fqa_sample's rule for the LDS copy of its boundary bin (copy_fits,
-flashqwen_amd/csrc/fqa_sample_select.h), run on the host by tests/cpp/sample_select.cpp with a
-restatement of the sums and the histogram before it: where the rule lets the bin be copied,
-every weight of the bin fits the copy's 16384 places."""
+"""fqa_sample's rules for what it counts and copies in LDS (flashqwen_amd/csrc/
+fqa_sample_select.h), run on the host by tests/cpp/sample_select.cpp.  copy_fits, behind a
+restatement of the sums and the histogram before it: where the boundary bin may be copied,
+every weight of the bin fits the copy's 16384 places.  in_columns: a weight counted in a
+level-1 column has one, NaNs too."""
 from __future__ import annotations
 
 import subprocess
@@ -45,12 +46,16 @@ def select(tmp_path_factory):
     if not Path(fb.HIPCC).exists():
         pytest.skip("hipcc not present")
     exe = tmp_path_factory.mktemp("select") / "sample_select"
-    # no contraction: the kernel rounds each product and sum (fmaf is written where it is meant)
-    subprocess.run([fb.HIPCC, "-O1", "-std=c++17", "-Wall", "-ffp-contract=off", "-x", "hip",
+    # no contraction: the kernel rounds each product and sum (fmaf is written where it is
+    # meant); no NaN semantics, as the library is built
+    subprocess.run([fb.HIPCC, "-O1", "-std=c++17", "-Wall", "-ffp-contract=off",
+                    "-fno-honor-nans", "-x", "hip",
                     "--offload-host-only", str(ROOT / "tests" / "cpp" / "sample_select.cpp"),
                     "-o", str(exe)], check=True, capture_output=True, text=True)
 
-    def run(lg, top_p):
+    def run(lg, top_p=()):
+        if lg is None:
+            return subprocess.run([str(exe), "columns"], capture_output=True, text=True)
         r = subprocess.run([str(exe), str(len(lg)), *(repr(float(t)) for t in top_p)],
                            input=lg.astype(np.float32).tobytes(), capture_output=True, check=True)
         return [tuple(map(int, line.split())) for line in r.stdout.decode().splitlines()]
@@ -78,3 +83,8 @@ def test_copied_bins_fit(select, vocab):
             assert fits == (counted <= CAP)
             copied += fits
     assert copied > 0
+
+
+def test_counted_weights_have_a_column(select):
+    r = select(None)
+    assert r.returncode == 0, r.stdout

@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
     __syncthreads();
     float above;
     int b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
-    if (b1 < kCol0) {
+    if (b1 < kCol0 && x_min < kBelowCols) {
       // the boundary lies further down (top_p within 2^-31 or so of 1, or rounding): the
       // bins below the columns too
       for_chunks([&](const Chunk& x, int) {
@@ -328,7 +328,10 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
       b1 = find_crossing(hist, kBins, 0.f, need, sh, &sres, &sres_f, &above);
     }
     const int e1 = b1 >> 3;  // the exponent field of every weight in bin b1
-    const bool copy = copy_fits(hcnt[b1], b1, x_min);
+    // Bin 0 holds no counted weight: it means that there is no boundary (top_p so near to 1
+    // that fp32 sums do not reach top_p * Z), and every weight is kept.
+    const bool all = b1 == 0;
+    const bool copy = all || copy_fits(hcnt[b1], b1, x_min);
     // pass 3: per lane, the mass of the weights above bin b1 (all kept), and the weights in
     // bin b1 copied into LDS (low 20 bits and the wave), on which level 2 (bits 19..9),
     // level 3 and the kept masses run without reading the row again; or level 2 here.
@@ -351,7 +354,7 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
           km1 += bb > b1 ? wv : 0.f;
           n += bb == b1 ? 1 : 0;
         }
-      if (!__any(n > 0)) return;
+      if (all || !__any(n > 0)) return;
       if (copy) {
         // room for this lane's n weights: one addition per wave; then without branches,
         // what is not copied goes to a spare word

@@ -21,6 +21,8 @@ __host__ __device__ inline float bin_mass(unsigned long long sum, int exp_field)
 
 constexpr int kCols = 256;  // level-1 bins with a column per lane: the 31 octaves below 1
 constexpr int kCol0 = (127 << 3) + 8 - kCols;  // ... from this bin on (bits 30..20)
+constexpr float kBelowCols = 0x1p-31f;  // weights below this lie below the columns
+static_assert(kCol0 == (127 - 31) << 3, "kBelowCols");
 
 // Whether a weight is counted in a column.  A NaN (of a NaN or infinite logit) has a bin past
 // the columns, and compiled without NaN semantics the comparison with x_min may let it pass.

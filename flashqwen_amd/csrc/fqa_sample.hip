@@ -16,19 +16,20 @@
 // row is read 3 times in full (max + sum, level 1, and a pass that copies the weights of the
 // boundary bin into LDS, on which levels 2 and 3 run).  Only when the boundary bin may hold
 // more than 16384 weights (copy_fits) is the row read a 4th time for level 3, and once more
-// where the boundary lies below 2^-31 of the largest weight.  A temperature-only row is read once (its
-// kept mass per wave is the rescaled pass-1 sum); the pick then reads 1/16 of one wave's
-// segment.
+// where the boundary lies below 2^-31 of the largest weight.  A temperature-only row is read
+// once (its kept mass per wave is the rescaled pass-1 sum); the pick then reads 1/16 of one
+// wave's segment.
 //
-// What bounds it: with a workgroup per row, what one CU loads and computes.  Each wave keeps
-// 4 KiB of loads in flight while it works on the 4 KiB before (128 KiB per CU; 2 KiB with no
-// overlap made a pass ~20 us however few the rows), and per-element work is kept free of
-// branches and of atomics that meet: the running maximum is selected, not branched on, level
-// 1 has a column per lane, room in the copy is taken once per 4 KiB.  Sums keep one order
-// (lane, step, element; then lanes; then waves), so a draw near a cumulative-mass boundary
-// falls the same way.  151936 logits, 4 rows: greedy 21.6 -> 13.7 us, temperature 27.6 -> 20.1,
-// top-p 0.9 71 -> 61, nearly flat rows 185 -> 76; 256 rows: 32.7 -> 32.0, 37.4 -> 36.6, 93 ->
-// 93 (HBM and the caches carry the reads there), 207 -> 115.
+// What bounds it: with a workgroup per row, what one CU loads and computes.  Each wave keeps a
+// chunk of loads in flight while it works on the one before (4 KiB of them, 128 KiB per CU,
+// where rows are few: 2 KiB with no overlap made a pass ~20 us however few the rows), and
+// per-element work is kept free of branches and of atomics that meet: the running maximum is
+// selected, not branched on, level 1 has a column per lane, room in the copy is taken once per
+// chunk.  Sums keep one order (lane, step, element; then lanes; then waves) whatever the chunk,
+// so a draw near a cumulative-mass boundary falls the same way.  151936 logits, 4 rows, before
+// and after: greedy 21.6 -> 13.1 us, temperature 27.6 -> 18.6, top-p 0.9 79.2 -> 60.4, nearly flat rows
+// 200.6 -> 74.8, masked rows (999 of 1000 at -inf) 51.7 -> 49.2; 256 rows (HBM and the caches
+// carry the reads) 27.4 -> 25.6, 33.1 -> 29.0, 91.2 -> 82.0, 212.3 -> 100.8, 77.0 -> 76.8.
 #include "fqa_common.h"
 #include "fqa_sample_select.h"
 
@@ -40,7 +41,6 @@ namespace {
 constexpr int kSThreads = 1024;
 constexpr int kSWaves = kSThreads / kWave;
 constexpr int kBins = 2048;  // histogram bins per radix level (levels use 11, 11, 9 bits)
-constexpr int kChunk = 4;    // 256-element steps whose loads a wave issues back to back
 
 struct SampArgs {
   const float* logits;
@@ -119,9 +119,17 @@ __device__ __forceinline__ void load4(const float* lg, int i, int end, float (&x
   }
 }
 
-typedef float Chunk[kChunk][4];
-
+// kChunk: 256-element steps whose loads a wave issues back to back and then works on (times:
+// top-p 0.95, normal logits; masked: 999 of 1000 at -inf).
+//  * 1 for rows of 16384 logits or less, which give a wave 4 steps at most, so that little of
+//    a chunk lies past the row's end: 1000 / 4000 / 16000 logits 13.4 / 14.4 /
+//    18.7 us against 15.5 / 17.8 / 18.5 with 4.
+//  * 2 above 128 rows, where the caches carry the reads: 151936 logits, 200 / 256 rows 74.6 /
+//    82.5 us against 76.8 / 87.9 with 4, 256 masked rows 76.5 against 80.4.
+//  * 4 otherwise: 4 / 64 / 128 rows 60.8 / 66.1 / 68.7 us against 61.8 / 68.8 / 70.0 with 2.
+template <int kChunk>
 __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
+  typedef float Chunk[kChunk][4];
   __shared__ float sh[kSWaves];
   __shared__ float sh2[kSWaves];
   __shared__ int sres;
@@ -145,9 +153,25 @@ __global__ void __launch_bounds__(kSThreads) sample_kernel(SampArgs a) {
     if (c0 + kSpan <= end) {
 #pragma unroll
       for (int u = 0; u < kChunk; ++u) __builtin_memcpy(x[u], lg + c0 + u * kStep + 4 * lane, 16);
-    } else {
+      return;
+    }
+    // the chunk that the end cuts: no branches by lane, which would wait for one load before
+    // the next
 #pragma unroll
-      for (int u = 0; u < kChunk; ++u) load4(lg, c0 + u * kStep + 4 * lane, end, x[u]);
+    for (int u = 0; u < kChunk; ++u) {
+      const int s0 = c0 + u * kStep, i = s0 + 4 * lane;
+      if (s0 + kStep <= end) {
+        __builtin_memcpy(x[u], lg + i, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[u][e] = -INFINITY;
+        if (s0 < end)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = lg[min(i + e, end - 1)];
+            x[u][e] = i + e < end ? v : -INFINITY;
+          }
+      }
     }
   };
   auto for_chunks = [&](auto&& f) {
@@ -589,7 +613,13 @@ extern "C" int fqa_sample(const float* logits, int32_t n_rows, int32_t vocab,
   if (n_rows == 0) return FQA_OK;
   if (!logits || !inv_temp || !top_p || !u || !out) return FQA_EINVAL;
   SampArgs a{logits, vocab, row_stride, inv_temp, top_p, u, out};
-  hipLaunchKernelGGL(sample_kernel, dim3((unsigned)n_rows), dim3(kSThreads), 0,
-                     (hipStream_t)stream, a);
+  const dim3 grid((unsigned)n_rows), block(kSThreads);
+  const hipStream_t st = (hipStream_t)stream;
+  if (vocab <= 16384)
+    hipLaunchKernelGGL(sample_kernel<1>, grid, block, 0, st, a);
+  else if (n_rows > 128)
+    hipLaunchKernelGGL(sample_kernel<2>, grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL(sample_kernel<4>, grid, block, 0, st, a);
   return hipGetLastError() == hipSuccess ? FQA_OK : FQA_ELAUNCH;
 }

@@ -862,11 +862,14 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::
   int* s_pos = reinterpret_cast<int*>(lds + T::kBM * kTP);
   int* s_slot = s_pos + T::kBM;
   const int T_rows = min(p.meta[FQA_META_ROWS], a.M);
-  // the rows' positions and slots, loaded while the tile goes to LDS (-1: no such row)
+  // the rows' positions and slots, loaded while the tile goes to LDS (position -1: no such
+  // row; slot -1: nothing to append)
   int my_pos = -1, my_slot = -1;
   if (threadIdx.x < T::kBM && row0 + (int)threadIdx.x < T_rows) {
     my_pos = p.positions[row0 + threadIdx.x];
     my_slot = p.slots[row0 + threadIdx.x];
+    if (my_pos < 0 || my_pos >= p.rope_max_pos || my_slot < 0 || my_slot / kPage >= p.pool_pages)
+      my_slot = -1;
   }
   stage_tile<T>(lds, acc, wm, wn, lane);
   if (threadIdx.x < T::kBM) {
@@ -933,14 +936,11 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::
           *reinterpret_cast<uint2*>(d) = olo[b];
           *reinterpret_cast<uint2*>(d + 64) = ohi[b];
         }
-        if (is_k && pos_ok) {
-          const int slot = s_slot[rt[b]];
-          const long long page = slot / kPage;
-          if (slot >= 0 && page < p.pool_pages) {
-            uint16_t* kd = p.pool + run_offset(page, head - kHq) + (slot % kPage) * kD + 4 * j;
-            *reinterpret_cast<uint2*>(kd) = olo[b];
-            *reinterpret_cast<uint2*>(kd + 64) = ohi[b];
-          }
+        const int slot = s_slot[rt[b]];
+        if (is_k && slot >= 0) {
+          uint16_t* kd = p.pool + run_offset(slot / kPage, head - kHq) + (slot % kPage) * kD + 4 * j;
+          *reinterpret_cast<uint2*>(kd) = olo[b];
+          *reinterpret_cast<uint2*>(kd + 64) = ohi[b];
         }
       }
     }
@@ -951,18 +951,17 @@ __device__ void append_epilogue(const GemmArgs& a, char* lds, const typename T::
   constexpr int kRows = T::kBM / T::kWaves;
   static_assert(kRows <= kWave && kRows % kPage == 0, "a lane per row");
   const int rt = w * kRows + min(lane, kRows - 1);
-  const int pos = s_pos[rt], slot = s_slot[rt];
+  const int slot = s_slot[rt];
   const int tok = slot % kPage, lt = rt - tok;  // the page's first row, in the tile
-  // (a row without a position is no row, or one that the append skips)
-  const bool valid = lane < kRows && pos >= 0 && pos < p.rope_max_pos && slot >= 0 &&
-                     slot / kPage < p.pool_pages;
-  // A page whose rows all lie in the tile (and that the append kernel would write whole:
-  // same test) is written by its first row; any other row writes its own column.  Both
-  // give the same bytes.
-  bool whole = valid && lt >= 0 && lt + kPage <= T::kBM && row0 + lt + kPage <= T_rows;
-  if (whole)
-    whole = s_slot[lt] == slot - tok && s_slot[lt + kPage - 1] == slot - tok + kPage - 1 &&
-            s_pos[lt] >= 0 && s_pos[lt + kPage - 1] < p.rope_max_pos;
+  const bool valid = lane < kRows && slot >= 0;
+  // A page whose 16 rows all lie in the tile, each in its place, is written by its first row;
+  // any other row writes its own column.
+  const bool inside = valid && lt >= 0 && lt + kPage <= T::kBM;
+  const int* first = s_slot + (inside ? lt : 0);
+  int off = 0;  // (every read is on its way before the first is looked at)
+#pragma unroll
+  for (int i = 0; i < kPage; ++i) off |= first[i] ^ (slot - tok + i);
+  const bool whole = inside && off == 0;
   const int kvh0 = head0 - kHq - kHkv;
   // whole pages: lane l holds dims 2l, 2l+1 of each head
   for (uint64_t m = __ballot(whole && tok == 0); m; m &= m - 1) {

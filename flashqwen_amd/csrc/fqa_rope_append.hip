@@ -184,15 +184,13 @@ __global__ void __launch_bounds__(256) qknorm_rope_append_kernel(AppendArgs a) {
 
   // ---- v ------------------------------------------------------------------------------
   if (!page_ok) return;
-  // Full page: rows lead..lead+15 hold this page's tokens 0..15 (their slots are
-  // distinct and consecutive, so checking the first and the last suffices), and every
-  // one of them has a table row (positions run consecutively within a request).
+  // Full page: rows lead..lead+15 hold this page's tokens 0..15 and each has a table row, so
+  // that all 16 come to the same answer here (lane l of each looks at row lead + l % 16).
   const int lead = row - tok;
   bool full = lead >= 0 && lead + kPage <= T;
   if (full) {
-    const int base_slot = slot - tok;
-    full = a.slots[lead] == base_slot && a.slots[lead + kPage - 1] == base_slot + kPage - 1 &&
-           a.positions[lead] >= 0 && a.positions[lead + kPage - 1] < a.rope_max_pos;
+    const int r = lane % kPage, p = a.positions[lead + r];
+    full = __all(a.slots[lead + r] == slot - tok + r && p >= 0 && p < a.rope_max_pos);
   }
   if (full) {
     // The page's 16 rows share its V^T: row tok moves kv head tok/2, dims 64*(tok%2) ..

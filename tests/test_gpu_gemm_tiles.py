@@ -92,9 +92,11 @@ def test_gemm_smaller_workspace(gpu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,write_k,rows", [
-    (100, 64, 1, None),     # one k step: the 128-row tile's append epilogue
+    (40, 64, 1, None),      # one k step: the 128-row tile's append epilogue
+    (100, 64, 1, None),
     (129, 1024, 0, None),   # a slab's fp32 sums through the append kernel
-    (345, 1024, 0, None),   # 128 x 128 tiles
+    (300, 1024, 0, None),   # 128 x 128 tiles
+    (345, 1024, 0, None),
     (448, 1024, 1, 440),    # ... with the row count inside the last one
     (450, 1024, 1, 440),    # two planes of 256 x 128 tiles through the append kernel
     (700, 512, 1, 690),     # 256 x 128 tiles

@@ -122,3 +122,78 @@ def test_qkv_fused_rows_below_m(gpu, M, rows):
     pool equals the unfused path's byte for byte."""
     nb = _case(gpu, M, 1024, 0, seed=M + 7, rows=rows)
     assert nb == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", [
+    (64, 1024),   # the append kernel, 10 waves per row
+    (300, 64),    # 128 x 128 tiles' epilogue
+    (1100, 64),   # larger tiles' epilogue; unfused, 5 waves per row
+])
+@pytest.mark.parametrize("bad", ["position", "slot", "gap"])
+def test_page_with_a_row_that_is_not_appended(gpu, M, K, bad):
+    """Pages whose first and last rows are in place but one between has no table row, no page
+    in the pool, or another page's slot: every other row's v is stored whole, the place of
+    the row left out keeps what it held, on both paths."""
+    import torch
+
+    from flashqwen_amd import _lib
+    from flashqwen_amd.gemm import gemm, workspace_bytes
+    from flashqwen_amd.step import alloc_pool, make_dims, rope_tables
+
+    print(f"[qkv_bad_row] M={M} K={K} {bad}", flush=True)
+    lib, dims = _lib.load(), make_dims()
+    rng = np.random.default_rng(M)
+    P, max_pos = M // 16 + 3, 4096
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(torch.bfloat16).to(gpu)
+    w = (torch.from_numpy(rng.standard_normal((6144, K)).astype(np.float32)) * 0.03).to(
+        torch.bfloat16).to(gpu)
+    ones = torch.ones(128, device=gpu)
+    cos, sin = (torch.from_numpy(t).to(gpu) for t in rope_tables(max_pos))
+    pos, slots = np.arange(M, dtype=np.int32), np.arange(M, dtype=np.int32)
+    spare = (P - 2) * 16  # a page that no other row uses
+    for k, r in enumerate(range(7, M - 16, 16)):  # one row between the ends of every page
+        if bad == "position":
+            pos[r + k % 4] = max_pos + 1
+        elif bad == "slot":
+            slots[r + k % 4] = P * 16 + 3
+        elif k < 16:
+            slots[r + k % 4] = spare + k
+    valid = (pos < max_pos) & (slots < P * 16)
+    pos_t, slot_t = torch.from_numpy(pos).to(gpu), torch.from_numpy(slots).to(gpu)
+    meta = torch.zeros(16, dtype=torch.int32, device=gpu)
+    meta[_lib.META_ROWS] = M
+    qkv = torch.zeros((M, 6144), dtype=torch.bfloat16, device=gpu)
+    gemm(x, w, out=qkv)
+    v = qkv.view(torch.int16)[:, 5120:].cpu().numpy().reshape(M, 8, 128)
+    want = np.full((P, 8, 128, 16), 7, np.int16)
+    want[slots[valid] // 16, :, :, slots[valid] % 16] = v[valid]
+
+    def pool():
+        p = alloc_pool(P)[0]
+        p.view(torch.int16).fill_(7)
+        return p
+
+    def check(p, what):
+        got = p.view(torch.int16).cpu().numpy().reshape(P, 8, 2, 2048)[:, :, 1].reshape(
+            P, 8, 128, 16)
+        assert np.array_equal(got, want), (what, int((got != want).sum()))
+
+    args = (ones.data_ptr(), ones.data_ptr(), cos.data_ptr(), sin.data_ptr(), max_pos,
+            pos_t.data_ptr(), slot_t.data_ptr(), meta.data_ptr())
+    pool_a, pool_b, pool_c, qkv_a = pool(), pool(), pool(), torch.zeros_like(qkv)
+    nb = workspace_bytes(M, 6144, K)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=gpu)
+    _lib.check(lib.fqa_qkv_proj_append(
+        C.byref(dims), x.data_ptr(), K, w.data_ptr(), K, M, K, qkv_a.data_ptr(), *args,
+        pool_a.data_ptr(), P, 0, ws.data_ptr() if nb else None, nb, None), "fused")
+    if bad != "position":
+        _lib.check(lib.fqa_store_kv(C.byref(dims), qkv.data_ptr(), pos_t.data_ptr(),
+                                    slot_t.data_ptr(), meta.data_ptr(), M, pool_c.data_ptr(), P,
+                                    None), "store")
+        check(pool_c, "fqa_store_kv")
+    _lib.check(lib.fqa_qknorm_rope_append(C.byref(dims), qkv.data_ptr(), *args, M,
+                                          pool_b.data_ptr(), P, 0, None), "append")
+    torch.cuda.synchronize()
+    check(pool_b, "unfused")
+    check(pool_a, "fused")

@@ -1196,12 +1196,15 @@ int splits_allowed(int M, int N, int K, int64_t bytes) {
   return fit > 16 ? 16 : fit > s ? (int)fit : s;
 }
 
-template <class T, bool kNT>
-void launch_quad(const GemmArgs& a, bool f32, dim3 grid, hipStream_t st) {
-  if (f32)
-    hipLaunchKernelGGL((gemm_quad_kernel<T, kNT, true, false>), grid, dim3(T::kThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL((gemm_quad_kernel<T, kNT, false, false>), grid, dim3(T::kThreads), 0, st, a);
+// f(kNT) for an unsplit launch of a quad tile: one row tile of 128 columns streams W from HBM
+// (and on 128 x 128 takes K in segments).  Every form of a call goes by this rule, so that
+// fqa_gemm, fqa_gemm_argmax and the append's epilogue sum a shape in one order.
+template <class T, class F>
+void unsplit_quad(const GemmArgs& a, F&& f) {
+  if constexpr (T::kBN == 128) {
+    if (a.m_tiles == 1) return f(std::true_type{});
+  }
+  f(std::false_type{});
 }
 template <class T>
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t st) {
@@ -1210,10 +1213,13 @@ void launch_gemm(const GemmArgs& a, bool f32, hipStream_t st) {
   if constexpr (kIsQuad<T>) {
     if (a.splits > 1)
       hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, true>), grid, block, 0, st, a);
-    else if (T::kBN == 128 && a.m_tiles == 1)
-      launch_quad<T, T::kBN == 128>(a, f32, grid, st);
     else
-      launch_quad<T, false>(a, f32, grid, st);
+      unsplit_quad<T>(a, [&](auto nt) {
+        if (f32)
+          hipLaunchKernelGGL((gemm_quad_kernel<T, decltype(nt)::value, true, false>), grid, block, 0, st, a);
+        else
+          hipLaunchKernelGGL((gemm_quad_kernel<T, decltype(nt)::value, false, false>), grid, block, 0, st, a);
+      });
   } else if (f32) {
     hipLaunchKernelGGL((gemm_kernel<T, true>), grid, block, 0, st, a);
   } else {
@@ -1226,15 +1232,18 @@ void launch_argmax(const GemmArgs& a, hipStream_t st) {
   const dim3 block(T::kThreads);
   if constexpr (!kIsQuad<T>)
     hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, block, 0, st, a);
-  else if (T::kBN == 128 && a.m_tiles == 1)
-    hipLaunchKernelGGL((gemm_quad_kernel<T, T::kBN == 128, false, false, true>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, false, true>), grid, block, 0, st, a);
+    unsplit_quad<T>(a, [&](auto nt) {
+      hipLaunchKernelGGL((gemm_quad_kernel<T, decltype(nt)::value, false, false, true>), grid, block, 0, st, a);
+    });
 }
 template <class T>
 void launch_append(const GemmArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((gemm_quad_kernel<T, false, false, false, false, true>),
-                     dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(T::kThreads), 0, st, a);
+  const dim3 grid((unsigned)(a.m_tiles * a.n_tiles));
+  const dim3 block(T::kThreads);
+  unsplit_quad<T>(a, [&](auto nt) {
+    hipLaunchKernelGGL((gemm_quad_kernel<T, decltype(nt)::value, false, false, false, true>), grid, block, 0, st, a);
+  });
 }
 // A slab's launch; planes: fp32 into a.part also without a split.
 template <class T>

@@ -451,7 +451,10 @@ int fqa_sample(const float* logits, int32_t n_rows, int32_t vocab, int64_t row_s
  * elements, x, W and y 16-byte aligned, and every row start of x and W within 4 GiB of
  * its base.  Shapes with few output tiles may split K over several workgroups and need
  * `workspace` (16-byte aligned) of fqa_gemm_workspace_bytes(M, N, K) bytes (0: none;
- * its contents need no initialisation).  M = 0 is a no-op. */
+ * its contents need no initialisation).  Every workspace of that size or more gives the same
+ * bits.  For some shapes a smaller one is accepted too, down to the K split that brings plain
+ * tiles to the 256 CUs once: K is then split into fewer parts, slower, with the fp32 sums in
+ * another order.  M = 0 is a no-op. */
 int64_t fqa_gemm_workspace_bytes(int32_t M, int32_t N, int32_t K);
 int fqa_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy,
              int32_t M, int32_t N, int32_t K, int32_t y_f32, void* workspace,

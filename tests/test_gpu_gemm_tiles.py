@@ -91,6 +91,69 @@ def test_gemm_smaller_workspace(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (61, 2048, 8192),       # slabs with K split
+    (700, 4096, 12288),     # 256 x 256 tiles, K split
+    (160, 2048, 12288),
+    (100, 6144, 4096),
+    (480, 6144, 4096),
+])
+def test_gemm_larger_workspace(gpu, M, N, K):
+    """A workspace larger than fqa_gemm_workspace_bytes asks for changes no bit."""
+    import torch
+
+    from flashqwen_amd.gemm import gemm, workspace_bytes
+
+    n = workspace_bytes(M, N, K)
+    assert n > 0
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M)
+    x = torch.empty(M, K, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    w = torch.empty(N, K, dtype=torch.bfloat16, device=gpu).normal_(0.0, 0.02, generator=g)
+    ws = torch.empty(max(16 * M * N * 4, 2 * n), dtype=torch.uint8, device=gpu)
+    want = gemm(x, w, out_f32=True, workspace=ws[:n])
+    for size in (n + 16, ws.numel()):
+        assert torch.equal(gemm(x, w, out_f32=True, workspace=ws[:size]), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (300, 16640, 64),       # 192 x 256 tiles, ragged
+    (300, 16512, 64),       # 256 x 192
+    (385, 22016, 64),       # 256 x 256
+    (130, 16512, 64),       # 256 x 128, one row tile
+    (1025, 256, 64),        # past 1024 rows the workspace holds a pair per 256 columns, where
+    (1025, 3840, 64),       # the plan's own tiles are 128 columns wide: 256 x 256 instead
+    (1100, 2048, 256),      # ... and fqa_gemm splits K
+])
+def test_argmax_tiles(gpu, M, N, K):
+    """fqa_gemm_argmax on each tile, within an exactly sized workspace, against the fp32
+    logits of fqa_gemm (the same values where it needs no workspace, else float64 products
+    within fp32 rounding)."""
+    import torch
+
+    from flashqwen_amd import _lib
+    from flashqwen_amd.gemm import gemm, gemm_argmax, workspace_bytes
+
+    print(f"[argmax_tiles] M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M + N)
+    x = torch.empty(M, K, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    w = torch.empty(N, K, dtype=torch.bfloat16, device=gpu).normal_(0.0, 0.5, generator=g)
+    x[-1] = w[-1] * 8  # the last row peaks in the last column
+    n = int(_lib.load().fqa_gemm_argmax_workspace_bytes(M, N, K))
+    ws = torch.full((n + 4096,), 0x5A, dtype=torch.uint8, device=gpu)
+    got = gemm_argmax(x, w, workspace=ws[:n]).long()
+    assert torch.all(ws[n:] == 0x5A)
+    if workspace_bytes(M, N, K) == 0:
+        logits, tol = gemm(x, w, out_f32=True), 0.0
+    else:
+        logits, tol = x.double() @ w.double().T, 1e-4
+    assert torch.all(logits.gather(1, got[:, None])[:, 0] >= logits.max(1).values - tol)
+    assert int(got[-1]) == N - 1
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,K,write_k,rows", [
     (40, 64, 1, None),      # one k step: the 128-row tile's append epilogue
     (100, 64, 1, None),

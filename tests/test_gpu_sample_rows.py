@@ -45,6 +45,19 @@ def test_top_p_rows(gpu, vocab):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [4097, 151936])
+def test_top_p_near_one(gpu, vocab):
+    """The boundary far down the row's tail, and past what fp32 sums resolve."""
+    rng = np.random.default_rng(vocab + 2)
+    B = 24
+    lg = _rows(rng, B, vocab)
+    tp = rng.choice([0.9995, 0.9999, 0.99999, 0.999999], size=B).astype(np.float32)
+    it, u = np.ones(B, np.float32), rng.random(B).astype(np.float32)
+    exact = _check_sampled(lg, it, tp, u, _run(lg, it, tp, u))
+    assert exact >= B - 2
+
+
+@pytest.mark.gpu
 def test_rows_on_four_bytes(gpu):
     """A row stride that is odd in elements: the 16-byte loads start on any 4 bytes."""
     import torch

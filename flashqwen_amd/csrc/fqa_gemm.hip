@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(T::kThreads, 1) gemm_quad_kernel(GemmArgs a) {
 //    is refilled with its rows of step t + kSlots and (x blocks) its MFMAs issue, so nearly
 //    the whole ring stays in flight.
 //  * What bounds it: HBM for W and the launch at a few rows (o_proj at 6 rows 9.1 us against
-//    7.4 for its W stream alone), the rate at which a CU stages x from L2 above (~70 KB/us).
+//    7.4 for its W stream alone), the rate at which a CU stages x from L2 above (60-70 KB/us).
 //  * W cold, against the K-split tiles and their reduction: o_proj at 6 / 32 / 100 / 250 rows
 //    14.1 / 14.7 / 18.5 / 23.3 -> 8.9 / 10.6 / 14.7 / 19.4 us, qkv at 6 / 32 / 100 rows 15.6 /
 //    16.2 / 19.7 -> 11.2 / 12.8 / 17.6, down at 6 / 64 rows 27.3 / 32.1 -> 21.0 / 27.3.
@@ -1113,22 +1113,28 @@ struct GemmPlan {
   int bm, bn, splits, m_tiles, n_tiles;
 };
 
-// Chosen by a model of the time in us, fitted to measurements on 6144 x 4096, 4096 x 4096,
-// 24576 x 4096 and 4096 x 12288 at 6 to 2048 rows with W cold (within ~15% of each, and
-// nearly always the measured order):
+// Chosen by a model of the time in us, fitted to measurements with W cold on 6144 x 4096, 4096 x
+// 4096, 24576 x 4096 and 4096 x 12288 at 6 to 2048 rows (within ~15% of each, and nearly always
+// the measured order), and checked on 22 widths from 128 to 24576 by 128 to 12288 k at 1 to
+// 1024 rows (4554 shapes: the plan is 2.5% behind the best of all plans on average):
 //  * Tiles of 128 columns or more: 2.4 for the launch and, per round of 256 workgroups, 5 to
 //    start and store and, per step of 64 k, 1.29 (256 x 256), 1.03 (192 x 256, 256 x 192; 1.24
 //    with K split), 0.78 (256 x 128) or 0.45 (128 x 128; 0.58 with K split, 0.75 with a single
-//    row tile, whose W comes from HBM).  What decides between them is mostly how full the
-//    last round is: gate_up at 384 / 700 / 1000 / 1500 rows 90 / 154 / 178 / 260 us without
+//    row tile unsplit, whose W comes from HBM).  What decides between them is mostly how full
+//    the last round is: gate_up at 384 / 700 / 1000 / 1500 rows 90 / 154 / 178 / 260 us without
 //    the 192-wide tiles, 80 / 141 / 164 / 238 with them; qkv at 1500 rows 77 -> 68, down 139 ->
 //    127.
-//  * Slabs: 6, 1 per 70 KB that a workgroup stages and 1 per 4096 outputs of the tile (the
+//  * A K split by a multiple of four at up to 256 rows: 15% more per step, its workgroups
+//    meeting on the same HBM channels (down at 160 / 200 / 256 rows, 256 x 128, 8 parts 41.8 /
+//    42.7 / 47.2 us, 7 parts 35.4 / 37.2 / 39.7).
+//  * Slabs: 6, 1 per 64 KB that a workgroup stages and 1 per 4096 outputs of the tile (the
 //    sum over its waves); one round of workgroups; for x that fits an XCD's L2
 //    beside the W stream (3.5 MB: at 12288 k and 160 rows the slabs lose).
-//  * A K split adds the reduction: 2.5, 1 per split and 1 per million fp32 partials (8 MB).
-// Up to 128 rows with 160 column tiles or more (gate_up, lm_head) the smallest tile that
-// covers M streams W once at HBM's rate, and nothing is split.
+//  * A K split adds the reduction: 2.5 (3 to a slab), 1 per split and 1 per million fp32
+//    partials (8 MB).
+// Up to 128 rows with more than 128 column tiles (gate_up, lm_head), where K cannot be split
+// over the CUs left, the smallest tile that covers M streams W once at HBM's rate (18944 x 1024
+// at 4 / 64 rows 11.5 / 13.5 us, in 128 x 128 tiles 14.0 / 15.8).
 // max_splits bounds K splits; 1 (fqa_gemm_argmax, and shapes whose workspace is empty) also
 // leaves the slabs out, so that equal shapes sum in the same order.
 GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
@@ -1136,7 +1142,7 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
   auto make = [&](int tile, int bm, int bn, int s) {
     return GemmPlan{tile, bm, bn, s, (M + bm - 1) / bm, N / bn};
   };
-  if (M <= 128 && N / 128 >= 160)
+  if (M <= 128 && N / 128 > 128)
     return M > 64 ? make(kTileM, 128, 128, 1) : M > 32 ? make(kTileS, 64, 128, 1) : make(kTileT, 32, 128, 1);
   // the QKV width at 449..512 rows (where the call may split): the append kernel reads two
   // planes.  With the append in the epilogue of 128 x 128 tiles, rows on their own pages keep
@@ -1168,7 +1174,8 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
       const GemmPlan p = make(q.tile, q.bm, q.bn, s);
       const long long g = (long long)p.m_tiles * p.n_tiles * s;
       if (s > 1 && g > 256) break;
-      const float step = q.tile == kTileM && p.m_tiles == 1 ? 0.75f : s > 1 ? q.split_step : q.step;
+      float step = s > 1 ? q.split_step : q.tile == kTileM && p.m_tiles == 1 ? 0.75f : q.step;
+      if (s > 1 && s % 4 == 0 && M <= 256) step *= 1.15f;
       consider(p, 2.4f + (float)((g + 255) / 256) * ((float)((nst + s - 1) / s) * step + 5.f));
     }
   }
@@ -1179,7 +1186,7 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
       for (int s = 1; s <= 4 && s <= max_splits && s <= nst; s *= 2) {
         const GemmPlan p = make(kSlab0 + i, bm, bn, s);
         if ((long long)p.m_tiles * p.n_tiles * s > 256) break;
-        consider(p, 6.f + (bm + bn) * 2.f * K / s / 70e3f + bm * bn / 4096.f);
+        consider(p, (s > 1 ? 6.5f : 6.f) + (bm + bn) * 2.f * K / s / 64e3f + bm * bn / 4096.f);
       }
     }
   }

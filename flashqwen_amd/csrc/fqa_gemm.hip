@@ -1144,12 +1144,19 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits) {
   };
   if (M <= 128 && N / 128 > 128)
     return M > 64 ? make(kTileM, 128, 128, 1) : M > 32 ? make(kTileS, 64, 128, 1) : make(kTileT, 32, 128, 1);
-  // the QKV width at 449..512 rows (where the call may split): the append kernel reads two
-  // planes.  With the append in the epilogue of 128 x 128 tiles, rows on their own pages keep
-  // the few CUs that hold V busy after all others: QKV + append at 450 / 500 / 512 such rows
-  // 43.3 / 49.4 / 49.4 us, split 42.4 / 43.9 / 44.2; 512-token prompts 36.4 / 40.4 / 41.2, split
-  // 42.1 / 42.8 / 43.1.  At 448 own-page rows the epilogue takes 43.1, at 260 / 400 39 / 40.
-  if (N == kQkvStride && M > 448 && M <= 512 && max_splits > 1) return make(kTileH, 256, 128, 2);
+  // The QKV width at 489..512 rows of 4096 k or more, where the call may split: K in two, and
+  // the append kernel reads the two planes.  With the append in the epilogue of 128 x 128 tiles,
+  // decode rows on their own pages keep the few CUs that hold V busy after all others; prompts
+  // and fqa_gemm, which has to share the plan so that fused and unfused agree, are faster
+  // unsplit.  Split / unsplit, 4096 k (us):
+  //   rows               464          484          488          496          512
+  //   own pages      44.9 / 46.9  45.4 / 48.6  45.1 / 48.9  45.5 / 49.8  45.4 / 50.5
+  //   512-token prompts  43.9 / 38.3  44.1 / 39.5  44.0 / 40.0  44.2 / 40.4  44.2 / 41.2
+  //   fqa_gemm       40.5 / 36.2  41.0 / 37.9  40.8 / 37.8  40.8 / 38.3  40.6 / 38.8
+  // With fewer k the split costs more (512 rows of 3072 k: 39.0 / 41.2, 37.4 / 31.1, 33.7 / 29.0;
+  // of 1024 k: 27.9 / 25.4, 26.1 / 14.5, 22.5 / 12.5).
+  if (N == kQkvStride && M > 488 && M <= 512 && K >= 4096 && max_splits > 1)
+    return make(kTileH, 256, 128, 2);
   GemmPlan best{};
   float best_us = 3.4e38f;
   auto consider = [&](const GemmPlan& p, float us) {

@@ -161,7 +161,10 @@ def test_argmax_tiles(gpu, M, N, K):
     (300, 1024, 0, None),   # 128 x 128 tiles
     (345, 1024, 0, None),
     (448, 1024, 1, 440),    # ... with the row count inside the last one
-    (450, 1024, 1, 440),    # two planes of 256 x 128 tiles through the append kernel
+    (450, 1024, 1, 440),
+    (488, 4096, 0, None),
+    (489, 4096, 1, 480),    # two planes of 256 x 128 tiles through the append kernel
+    (512, 4032, 0, None),   # ... which take 4096 k or more
     (700, 512, 1, 690),     # 256 x 128 tiles
     (1500, 256, 0, 1490),   # 192 x 256 tiles
 ])
